@@ -16,6 +16,13 @@ from . import _hip
 from ._checks import require_cuda
 
 
+# from this many routes 256-token tiles (MI355X, 4,001 tokens: gate_up + down 1,182 us on 64-token
+# tiles, the whole call 1,151 -> 694), from this many rows the many-workgroup bucketing (40 us in
+# one workgroup there): the engine's own thresholds (dsv2lite.engine)
+BIG_TILE_ROUTES = 5120
+WIDE_BUCKET_MIN_ROWS = 1024
+
+
 @dataclass
 class PackedRoutedExperts:
     # gate_up_weights: [num_experts, 2 * intermediate_size, hidden_size] (per expert [gate; up])
@@ -100,7 +107,10 @@ def batched_grouped_routed_moe_grouped_triton(x: torch.Tensor, topk_ids: torch.T
         raise ValueError("batched_grouped_routed_moe supports at most 8192 tokens per call")
     dev = x.device
     avg = R / 64
-    tile = 16 if avg <= 6 else (32 if avg <= 16 else 64)
+    if R >= BIG_TILE_ROUTES and I % 128 == 0:
+        tile = 256
+    else:
+        tile = 16 if avg <= 6 else (32 if avg <= 16 else 64)
     max_tiles = math.ceil(R / tile) + 64
     sorted_routes = torch.empty(R, dtype=torch.int32, device=dev)
     route_pos = torch.empty(R, dtype=torch.int32, device=dev)
@@ -110,8 +120,13 @@ def batched_grouped_routed_moe_grouped_triton(x: torch.Tensor, topk_ids: torch.T
     ys = torch.empty(R, 2048, dtype=torch.bfloat16, device=dev)
     out = torch.empty(B, 2048, dtype=torch.bfloat16, device=dev)
     st = _hip.stream_ptr(dev)
-    _hip.call("dsv2_moe_bucket", ids.data_ptr(), B, tile, sorted_routes.data_ptr(), route_pos.data_ptr(),
-              tiles.data_ptr(), ntiles.data_ptr(), st)
+    if B >= WIDE_BUCKET_MIN_ROWS:
+        ws = torch.empty(_hip.lib.dsv2_moe_bucket_workspace_size(B), dtype=torch.uint8, device=dev)
+        _hip.call("dsv2_moe_bucket_wide", ids.data_ptr(), B, tile, sorted_routes.data_ptr(), route_pos.data_ptr(),
+                  tiles.data_ptr(), ntiles.data_ptr(), ws.data_ptr(), ws.numel(), st)
+    else:
+        _hip.call("dsv2_moe_bucket", ids.data_ptr(), B, tile, sorted_routes.data_ptr(), route_pos.data_ptr(),
+                  tiles.data_ptr(), ntiles.data_ptr(), st)
     _hip.call("dsv2_moe_grouped_gateup", x.data_ptr(), sorted_routes.data_ptr(), tiles.data_ptr(), ntiles.data_ptr(),
               max_tiles, tile, packed.gate_up_weights.data_ptr(), I, hs.data_ptr(), st)
     _hip.call("dsv2_moe_grouped_down", hs.data_ptr(), tiles.data_ptr(), ntiles.data_ptr(), max_tiles, tile,

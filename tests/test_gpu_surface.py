@@ -399,6 +399,31 @@ def test_batched_attention_decode_q1_expanded_vs_fp32(B, H, L, pos, Dq, Dv):
         check_expanded_status(DEV)
 
 
+@pytest.mark.parametrize("tokens", [853, 854, 1024])
+def test_grouped_moe_wrapper_tile_threshold(tokens):
+    """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds,
+    experts unevenly loaded (one empty), against fp32 torch; three bf16 roundings (SwiGLU, expert
+    output, sum) of about 2^-9 each: 1e-2."""
+    from triton_kernels.moe_batch import PackedRoutedExperts, batched_grouped_routed_moe
+
+    I = 128
+    gu, dn = rnd(64, 2 * I, 2048, seed=80, std=0.02), rnd(64, 2048, I, seed=81, std=0.05)
+    x = rnd(tokens, 2048, seed=82)
+    g = torch.Generator().manual_seed(83)
+    logits = torch.randn(tokens, 64, generator=g) + torch.linspace(-2, 2, 64)
+    logits[:, 5] = -1e9
+    w, ids = torch.softmax(logits, -1).topk(6, -1)
+    out = batched_grouped_routed_moe(x, ids.to(DEV), w.to(DEV), PackedRoutedExperts(gu, dn, 2048, I, 64, 6))
+    ref = torch.zeros(tokens, 2048)
+    xc = c(x)
+    for e in range(64):
+        r, s = (ids == e).nonzero(as_tuple=True)
+        if r.numel():
+            h = xc[r] @ c(gu[e]).t()
+            ref.index_add_(0, r, (torch.nn.functional.silu(h[:, :I]) * h[:, I:]) @ c(dn[e]).t() * w[r, s, None])
+    assert rel_err(c(out), ref) < 1e-2
+
+
 # --------------------------------------------------------------------------- capacity guard (C ABI)
 def test_mla_kernels_never_touch_another_rows_slots():
     """Row 0 at pos == cap (full), row 1 with room.  The split-KV path (prepare + decode +
