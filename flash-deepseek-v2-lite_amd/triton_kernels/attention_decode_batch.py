@@ -227,11 +227,25 @@ def batched_attention_decode_q1_triton(query_states: torch.Tensor, key_states: t
     if B == 0 or L == 0:
         return out
     q, k, v = query_states, key_states, value_states
-    _hip.call("dsv2_attention_decode_expanded", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0),
+    ns = expanded_splits(B * H, L)
+    part = torch.empty(B, H, ns, Dv + 2, dtype=torch.float32, device=q.device) if ns > 1 else None
+    _hip.call("dsv2_attention_decode_expanded_split", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0),
               k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(),
-              out.stride(0), out.stride(1), B, H, Dq, Dv, L, cache_position.data_ptr(), float(softmax_scale),
-              _expanded_status(q.device).data_ptr(), _hip.stream_ptr(q.device))
+              out.stride(0), out.stride(1), B, H, Dq, Dv, L, cache_position.data_ptr(), float(softmax_scale), ns,
+              _hip.ptr(part), _expanded_status(q.device).data_ptr(), _hip.stream_ptr(q.device))
     return out
+
+
+def expanded_splits(pairs: int, length: int) -> int:
+    """Token ranges per (row, head) of the expanded-cache attention: several only where the
+    pairs leave most CUs idle and the cache is long enough to pay for the merge launch and its
+    buffer.  Measured on MI355X (whole calls, one range against the best of 2..16; pairs x cached
+    tokens): 16 x 4000 49.2 -> 20.9 us with 8, 32 x 3000 40.7 -> 21.3 with 8, 64 x 3900 53.2 ->
+    33.0 with 4; but 16 x 900 16.3 -> 20.3, 64 x 800 15.4 -> 19.6, 128 x 2000 33.3 -> 32.4 and
+    192 x 1380 29.2 -> 35.9."""
+    if pairs > 96 or length < 1536:
+        return 1
+    return max(1, min(8, length // 512, 256 // max(pairs, 1)))
 
 
 _EXPANDED_STATUS: dict = {}

@@ -286,6 +286,16 @@ int dsv2_attention_decode_expanded(const void* q, int64_t q_stride_b, int64_t q_
                                    int v_dim, int seq_len, const int64_t* cache_position, float softmax_scale,
                                    int32_t* status, void* stream);
 
+/* dsv2_attention_decode_expanded with each (row, head)'s tokens cut into `splits` (1..64)
+ * ranges of whole 32-token passes, for few (row, head) pairs over long caches; a second launch
+ * merges them in order.  workspace: fp32 [B, H, splits, v_dim + 2], unused for splits = 1. */
+int dsv2_attention_decode_expanded_split(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* k,
+                                         int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_s, const void* v,
+                                         int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s, void* out,
+                                         int64_t out_stride_b, int64_t out_stride_h, int batch, int heads, int q_dim,
+                                         int v_dim, int seq_len, const int64_t* cache_position, float softmax_scale,
+                                         int splits, float* workspace, int32_t* status, void* stream);
+
 /* Prefill attention (the prompt's tokens, before the decode path) in MLA's expanded form,
  * per head h and query row r (position p, in the sequence whose position 0 is cache row sb):
  *   out[r, h*128 + i] = bf16( softmax_{n <= p}(scale * q_rh . k_nh) . v_nh[i] )

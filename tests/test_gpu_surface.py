@@ -399,6 +399,28 @@ def test_batched_attention_decode_q1_expanded_vs_fp32(B, H, L, pos, Dq, Dv):
         check_expanded_status(DEV)
 
 
+@pytest.mark.parametrize("B,H,L,pos,Dq,Dv", [
+    (1, 2, 1, 0, 8, 8),            # one token, one chunk
+    (2, 3, 33, 31, 192, 128),      # the last of a group's four tokens
+    (2, 3, 300, 256, 200, 136),    # a ragged chunk, one token past a workgroup pass
+    (1, 4, 600, 288, 256, 256),    # the widest rows
+    (1, 16, 1536, 1535, 192, 128),  # split: every range full
+    (2, 16, 4096, 700, 192, 128),  # split: ranges without a token
+])
+def test_expanded_attention_tile_edges(B, H, L, pos, Dq, Dv):
+    """Edges of the wave passes and splits against fp64; the result is one bf16 round (2^-9) of an
+    fp32 sum, so 4e-3 relative bounds it with room for the fp32 exponentials."""
+    from triton_kernels.attention_decode_batch import batched_attention_decode_q1_triton
+
+    q, k, v = rnd(B, H, 1, Dq, seed=73), rnd(B, H, L, Dq, seed=74), rnd(B, H, L, Dv, seed=75)
+    k[:, :, pos + 1:] = float("nan")  # rows past the position are not read
+    v[:, :, pos + 1:] = float("inf")
+    out = batched_attention_decode_q1_triton(q, k, v, torch.tensor([pos], device=DEV), 0.1147)
+    kd, vd = k[:, :, :pos + 1].double().cpu(), v[:, :, :pos + 1].double().cpu()
+    s = (kd @ q.double().cpu().transpose(2, 3)).transpose(2, 3) * 0.1147
+    assert rel_err(c(out), torch.softmax(s, -1) @ vd) < 4e-3
+
+
 @pytest.mark.parametrize("tokens", [853, 854, 1024])
 def test_grouped_moe_wrapper_tile_threshold(tokens):
     """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds,
