@@ -29,13 +29,16 @@ static inline bool dsv2_aligned16(const void* p) { return (reinterpret_cast<uint
 // ---- bf16 <-> fp32 ---------------------------------------------------------
 __device__ __forceinline__ float bf2f(bf16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
-// round-to-nearest-even, NaN kept quiet (torch's float->bfloat16 conversion)
-__device__ __forceinline__ bf16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<bf16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<bf16_t>(u >> 16);
+// round-to-nearest-even, NaN kept quiet (torch's float->bfloat16 conversion), by gfx950's
+// v_cvt_pk_bf16_f32: the integer form (NaN test, round bit, add, shift) it stands for took six
+// VALU instructions per value; both give the same bits for all 2^32 inputs (checked on MI355X)
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float floatx2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  const floatx2_t v = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
+__device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, static_cast<__bf16>(f)); }
 
 // value of f after rounding to bf16, as fp32
 __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
@@ -49,10 +52,6 @@ __device__ __forceinline__ void unpack8(const uint4& v, float* f) {
   f[5] = __uint_as_float(v.z & 0xffff0000u);
   f[6] = __uint_as_float(v.w << 16);
   f[7] = __uint_as_float(v.w & 0xffff0000u);
-}
-
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  return static_cast<uint32_t>(f2bf(lo)) | (static_cast<uint32_t>(f2bf(hi)) << 16);
 }
 
 __device__ __forceinline__ uint4 pack8(const float* f) {

@@ -744,7 +744,6 @@ constexpr int kF8Wgs32 = 768, kF8Wgs64 = 512;
 // 8 e4m3 bytes -> 8 bf16 by v_cvt_scalef32_pk_bf16_fp8 (two per instruction, scale 1: an e4m3
 // value is a bf16 value, so the conversion is exact; the row scale is applied in fp32 later)
 __device__ __forceinline__ bf16x8_t fp8x8_to_bf16x8(uint32_t w0, uint32_t w1) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
   const bf16x2_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false);
   const bf16x2_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true);
   const bf16x2_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false);

@@ -26,7 +26,6 @@ namespace {
 constexpr int kAttWaves = 8, kAttTB = 2;  // tokens per 16-lane row per batch (p.v pairs them)
 constexpr int kAttRows = kAttWaves * 4;   // 16-lane rows per workgroup
 constexpr int kAttStep = kAttWaves * 4 * kAttTB;  // tokens per workgroup per batch
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float dot2bf(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
