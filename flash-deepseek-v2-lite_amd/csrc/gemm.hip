@@ -437,19 +437,9 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs& a, int g, int slot, 
 constexpr int kDmaStages = 4;
 constexpr int kDmaGroupedWgs = 512;  // 256 CUs x 2 (64 KB of LDS each)
 
-// xcd_blocked (the prefill shape): the work items, token-tile-major (all feature blocks of a
-// token tile, then the next tile, an expert's tiles in a row), are cut into 8 contiguous
-// ranges, one per XCD (workgroup i runs on XCD i % 8), and every item reads its K chunks in
-// order.  The ~32 items an XCD runs at once then share each token chunk among the tile's
-// feature blocks and each weight chunk among the expert's tiles in that XCD's L2; the decode
-// order instead puts all token tiles of a feature block on one XCD, which at prefill sizes
-// (token rows 3x the weight bytes) re-reads every token row from HBM on every XCD
-// (8192 x 2048 x 2048: 80.4 -> 74.2 us; C3 prefill 4.27 -> 4.15 s).
 struct DmaShape {
   int tiles, nwg, nfb;
-  int xcd_blocked;
 };
-
 
 // SWIGLU: the 64 weight rows of a workgroup are, per 16 features, 16 gate rows then the 16
 // matching up rows (32 features per workgroup); a wave's two row blocks are then one
@@ -458,11 +448,12 @@ struct DmaShape {
 // the live (tile, feature block) items only, so the table's dead tiles cost no workgroup
 // launches; token rows are gathered through slot_row and the tile's expert selects the
 // weights.
-template <bool SWIGLU, int WM = 32, int WN = 32, int ST = kDmaStages, int RWV = 2>
-__global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, const DmaShape sh) {
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) void gemm_dma_kernel(const GemmArgs a, const DmaShape sh) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];  // ST stages of SB bytes
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
-  constexpr int NW = 2 * RWV;                // waves: RWV along the weight rows x 2 along the tokens
+  constexpr int WM = 32, WN = 32, ST = kDmaStages;
+  constexpr int RWV = 2, NW = 2 * RWV;       // waves: RWV along the weight rows x 2 along the tokens
   constexpr int TM = RWV * WM, TN = 2 * WN;  // weight rows, tokens per workgroup
   constexpr int KC = 64, RB = 2 * KC;        // K per chunk; a chunk's bytes per row (8 pieces of 16 B)
   constexpr int RPL = 8;                     // rows per ring load (64 lanes x 16 B)
@@ -470,7 +461,7 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
   constexpr int LW = TM / (RPL * NW), LL = (TM + TN) / (RPL * NW);  // ring loads per wave per chunk: weights, all
   constexpr int XM = WM / 16, XN = WN / 16;  // MFMA blocks per wave
   constexpr int FPW = SWIGLU ? TM / 2 : TM;  // output features per workgroup
-  static_assert(LL <= 8 && XM <= 4 && XN <= 8, "local arrays have literal sizes");
+  static_assert(LL == 4 && XM == 2 && XN == 2, "local arrays have literal sizes");
   // piece p of row r sits in slot p ^ (r & 7): the 16 rows one MFMA fragment reads hit
   // distinct banks in every group of 8 lanes
   auto swz = [](int r) { return r & 7; };
@@ -483,14 +474,7 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
     int fb, g = 0, t0, count;
     bool shared = false;
     if (a.tiles) {
-      int j;
-      if (sh.xcd_blocked) {  // XCD blockIdx % 8 runs items [x * per, (x + 1) * per)
-        const int per = (live * sh.nfb + 7) / 8, jl = blockIdx.x / 8 + it * (gridDim.x / 8);
-        if (jl >= per) break;
-        j = (blockIdx.x % 8) * per + jl;
-      } else {
-        j = blockIdx.x + it * gridDim.x;
-      }
+      const int j = blockIdx.x + it * gridDim.x;
       if (j >= live * sh.nfb) break;
       const int tile = j / sh.nfb;
       fb = j % sh.nfb;
@@ -510,8 +494,8 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
       const int per = sh.nwg / 8;
       const int w = (blockIdx.x % 8) * per + blockIdx.x / 8;
       if (w >= sh.nfb * sh.tiles) break;
-      const int tile = sh.xcd_blocked ? w / sh.nfb : w % sh.tiles;
-      fb = sh.xcd_blocked ? w % sh.nfb : w / sh.tiles;
+      const int tile = w % sh.tiles;
+      fb = w / sh.tiles;
       t0 = tile * TN;
       count = min(TN, a.rows - t0);
     }
@@ -523,8 +507,8 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
     const bf16_t* const wbase = shared ? a.W2 + g * a.w2g : a.W + g * a.wg;
     const int64_t wld = shared ? a.w2ld : K;
     const int upoff = shared ? a.w2up : a.N;
-    const bf16_t* src[8];
-    int dst[8];
+    const bf16_t* src[4];
+    int dst[4];
 #pragma unroll
     for (int j = 0; j < LL; ++j) {
       const bool tok = j >= LW;
@@ -545,14 +529,15 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
       }
       dst[j] = (tok ? TM * RB + ((TN / NW) * wv + RPL * (j - LW)) * RB : ((TM / NW) * wv + RPL * j) * RB);
     }
-    // the item's K chunks start at a rotation that spreads the workgroups' concurrent requests
-    // over the weight rows' address range instead of one column of 128 B lines (C3 grouped
-    // gate_up 158.4 -> 153.6 us).  It depends on (expert or shared half, feature block) only:
-    // an expert's results do not depend on which other tiles share the launch, and the token
-    // tiles of one weight block read its chunks in the same order, so the ones that run
+    // grouped: the item's K chunks start at a rotation that spreads the workgroups' concurrent
+    // requests over the weight rows' address range instead of one column of 128 B lines (C3
+    // grouped gate_up 158.4 -> 153.6 us).  It depends on (expert or shared half, feature block)
+    // only: an expert's results do not depend on which other tiles share the launch, and the
+    // token tiles of one weight block read its chunks in the same order, so the ones that run
     // together share each chunk's fetch in L2 (a rotation per token tile as well made the
-    // reference workload at bsz=256 -- 4 tiles per expert -- 1.5x slower)
-    const int rot = sh.xcd_blocked ? 0 : (int)((unsigned)(fb * 7 + g * 13 + (shared ? 3 : 0)) % (unsigned)nch);
+    // reference workload at bsz=256 -- 4 tiles per expert -- 1.5x slower).  Dense launches take
+    // their chunks in order: each output then is the same sum, bit for bit, as gemm_big_kernel's
+    const int rot = a.tiles ? (int)((unsigned)(fb * 7 + g * 13 + (shared ? 3 : 0)) % (unsigned)nch) : 0;
     auto issue = [&](int chunk, int buf) {
       int cc = min(chunk, nch - 1) + rot;  // past the last chunk: repeat it (never multiplied)
       if (cc >= nch) cc -= nch;
@@ -561,7 +546,7 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
         __builtin_amdgcn_global_load_lds(src[j] + cc * KC,
                                          (__attribute__((address_space(3))) void*)(lds + buf * SB + dst[j]), 16, 0, 0);
     };
-    floatx4_t acc[4][8];
+    floatx4_t acc[2][2];
 #pragma unroll
     for (int x = 0; x < XM; ++x)
 #pragma unroll
@@ -600,39 +585,12 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if constexpr (ST == 2 && XM == 4 && XN == 8 && LL == 8) {
-          // the prefill shape: the next chunk's 8 ring loads go out one per 4 MFMAs of the
-          // first sub-step (sched_barrier pins the order) instead of as one burst that holds
-          // up the wave's MFMA issue (8192 x 2816 x 2048: 132.3 -> 121.7 us)
-          int cc = min(c + 1, nch - 1) + rot;
-          if (cc >= nch) cc -= nch;
-          const int buf = (i + 1) % ST;
-          bf16x8_t af[4], bfr[8];
-          frags(lds + i * SB, 0, af, bfr);
+        issue(c + ST - 1, (i + ST - 1) % ST);
 #pragma unroll
-          for (int x = 0; x < XM; ++x)
-#pragma unroll
-            for (int y = 0; y < XN; ++y) {
-              acc[x][y] = mfma16x16x32(af[x], bfr[y], acc[x][y]);
-              if (y % 4 == 3) {
-                const int j = x * 2 + y / 4;
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_global_load_lds(src[j] + cc * KC,
-                                                 (__attribute__((address_space(3))) void*)(lds + buf * SB + dst[j]),
-                                                 16, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-              }
-            }
-          frags(lds + i * SB, 1, af, bfr);
+        for (int s = 0; s < KC / 32; ++s) {
+          bf16x8_t af[2], bfr[2];
+          frags(lds + i * SB, s, af, bfr);
           mfmas(af, bfr);
-        } else {
-          issue(c + ST - 1, (i + ST - 1) % ST);
-#pragma unroll
-          for (int s = 0; s < KC / 32; ++s) {
-            bf16x8_t af[4], bfr[8];
-            frags(lds + i * SB, s, af, bfr);
-            mfmas(af, bfr);
-          }
         }
       }
     }
@@ -681,37 +639,366 @@ __global__ __launch_bounds__(RWV * 128) void gemm_dma_kernel(const GemmArgs a, c
   }
 }
 
-// grouped: max_tiles entries of a tile table of 64 (big: 256) tokens; dense: a.rows tokens.
-// big: 256 weight rows x 256 tokens per 8-wave workgroup (each wave 64 x 128, 4 x 8 MFMA
-// blocks), two 64 KB stages (a third does not fit the 160 KB of LDS), one workgroup per CU
-// -- for expert tiles of hundreds of tokens (prefill), where the 64 x 64 shape re-reads each
-// weight chunk once per 64 tokens and issues one MFMA per 2 KB of LDS reads (C3 prefill
-// 7.1 s -> 6.0 s with 128 x 128 per 4-wave workgroup, 5.3 s with 256 x 128 per 8 waves and
-// three 48 KB stages; with the later attention changes 4.76 s -> 4.43 s with 256 x 256).
-constexpr int kBigRwv = 4, kBigStages = 2, kBigWn = 128;  // big: waves along the weight rows, ring stages,
-constexpr int kBigTokens = 2 * kBigWn;                    // tokens per wave; tokens per workgroup
-constexpr int kBigRows = 64 * kBigRwv;                 // weight rows per big workgroup
-static void launch_dma(const GemmArgs& a, bool swiglu, hipStream_t st, int max_tiles = 0, bool big = false) {
+// grouped: max_tiles entries of a table of 64-token tiles; dense: a.rows tokens
+static void launch_dma(const GemmArgs& a, bool swiglu, hipStream_t st, int max_tiles = 0) {
   DmaShape sh;
-  sh.xcd_blocked = big;
-  const int tn = big ? kBigTokens : 64;
   // plain: a last feature block past N (N % 64 == 0) repeats row N-1 and stores nothing there
-  sh.nfb = swiglu ? a.N / (big ? kBigRows / 2 : 32) : (a.N + (big ? kBigRows : 64) - 1) / (big ? kBigRows : 64);
-  sh.tiles = a.tiles ? max_tiles : (a.rows + tn - 1) / tn;
-  // grouped: resident workgroups (two per CU, big: one) looping over the live items
-  sh.nwg = a.tiles ? (big ? kDmaGroupedWgs / 2 : kDmaGroupedWgs) : (sh.nfb * sh.tiles + 7) / 8 * 8;
-  if (big) {
-    constexpr int lds = kBigStages * (kBigRows + kBigTokens) * 128;
-    if (swiglu)
-      hipLaunchKernelGGL((gemm_dma_kernel<true, 64, kBigWn, kBigStages, kBigRwv>), dim3(sh.nwg),
-                         dim3(128 * kBigRwv), lds, st, a, sh);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<false, 64, kBigWn, kBigStages, kBigRwv>), dim3(sh.nwg),
-                         dim3(128 * kBigRwv), lds, st, a, sh);
-    return;
-  }
+  sh.nfb = swiglu ? a.N / 32 : (a.N + 63) / 64;
+  sh.tiles = a.tiles ? max_tiles : (a.rows + 63) / 64;
+  // grouped: resident workgroups (two per CU) looping over the live items
+  sh.nwg = a.tiles ? kDmaGroupedWgs : (sh.nfb * sh.tiles + 7) / 8 * 8;
   if (swiglu) hipLaunchKernelGGL(gemm_dma_kernel<true>, dim3(sh.nwg), dim3(256), kDmaStages * 16384, st, a, sh);
   else hipLaunchKernelGGL(gemm_dma_kernel<false>, dim3(sh.nwg), dim3(256), kDmaStages * 16384, st, a, sh);
+}
+
+// Large tiles (prefill): 256 weight rows (SwiGLU: 128 features, gate and up) x up to 256 tokens per
+// 4-wave workgroup, one workgroup per CU and one wave per SIMD, each wave 64 weight rows x all the
+// tile's tokens in 64 x NG / 16 MFMA blocks.  K goes in 64-wide chunks through two LDS stages
+// (64 KB each) filled by global_load_lds; each half chunk's fragments are read from LDS while the
+// previous half's MFMAs run, and the stage just read is refilled during the second half, so a chunk
+// costs one barrier and its loads have a chunk's time to land.  A persistent grid: the last pair of
+// chunks requests the next item's first two, whose latency the epilogue covers.  A tile of at most
+// 64 / 128 / 192 tokens runs a loop of that many (NG).  Every output is one accumulator's sum over
+// K in order, whatever NG.
+// The work items, token-tile-major (all feature blocks of a token tile, then the next tile, an
+// expert's tiles in a row), are cut into 8 contiguous ranges, one per XCD (workgroup i runs on XCD
+// i % 8): the ~32 items an XCD runs at once share each token chunk among the tile's feature blocks
+// and each weight chunk among the expert's tiles in that XCD's L2.
+// Bound: MFMA issue at the clock the power limit leaves (8192 x 10944 x 2048: 1.41 PFLOP/s at 1.88
+// GHz, MFMA busy 70%; hipBLASLt 1.57 at 1.74 GHz, 83%).  MI355X, against 8 waves of 64 x 128 (two
+// per SIMD) on one barrier and one burst of LDS reads per half chunk: 8192 x 2048 x 2048 67.5 ->
+// 63.4 us, x 2816 x 2048 88 -> 78, routed gate_up of 8,192 tokens 640 -> 600, down 385 -> 328.
+// Four waves of 128 x 128 read 20% less LDS but cannot skip a short tile's missing tokens.
+constexpr int kBigRows = 256, kBigTokens = 256, kBigStage = (kBigRows + kBigTokens) * 128, kBigWgs = 256;
+struct BigShape {
+  int tiles, nfb, tokens;  // token tiles (grouped: the table's size), feature blocks, dense: tokens per tile
+  bool wide;               // outputs and residual rows are 16-byte aligned
+};
+
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+// A work item: the weight rows and tokens of one output tile.
+struct BigItem {
+  int g, f0, t0, count;
+  bool shared;
+};
+
+__device__ __forceinline__ int big_items(const GemmArgs& a, const BigShape& sh) {
+  const int ns = a.W2 ? 2 * a.s_tiles : 0;
+  return (a.tiles ? ns + min(a.ntiles[0], sh.tiles) : sh.tiles) * sh.nfb;
+}
+
+template <bool SWIGLU>
+__device__ __forceinline__ BigItem big_item(const GemmArgs& a, const BigShape& sh, int j) {
+  BigItem it;
+  const int ns = a.W2 ? 2 * a.s_tiles : 0;
+  const int tile = j / sh.nfb;
+  it.f0 = (j % sh.nfb) * (SWIGLU ? kBigRows / 2 : kBigRows);
+  it.g = 0;
+  it.shared = false;
+  if (!a.tiles) {
+    it.t0 = tile * sh.tokens;
+    it.count = min(sh.tokens, a.rows - it.t0);
+  } else if (tile < ns) {
+    it.shared = true;
+    it.g = tile / a.s_tiles;
+    it.t0 = (tile % a.s_tiles) * kBigTokens;
+    it.count = min(kBigTokens, a.rows - it.t0);
+  } else {
+    const int4 tt = reinterpret_cast<const int4*>(a.tiles)[tile - ns];
+    it.g = tt.x;
+    it.t0 = tt.y;
+    it.count = min(tt.z, kBigTokens);
+  }
+  return it;
+}
+
+// Ring loads of this wave: weight load j covers weight rows 64 wv + 8 j .. + 7, token load j
+// tokens 8 (4 j + wv) .. + 7 (128 B of K each); lane -> (row, 16-byte slot lane & 7), which
+// holds piece (lane & 7) ^ (row & 7).
+struct BigSrc {
+  const bf16_t *w[8], *t[8];
+};
+
+template <bool SWIGLU>
+__device__ __forceinline__ void big_src(const GemmArgs& a, const BigItem& it, BigSrc& s) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r8 = lane >> 3, pc = ((lane & 7) ^ r8) * 8;
+  const bf16_t* const wbase = it.shared ? a.W2 + it.g * a.w2g : a.W + it.g * a.wg;
+  const int64_t wld = it.shared ? a.w2ld : a.K;
+  const int upoff = it.shared ? a.w2up : a.N;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {  // rows past N: row N - 1 (their outputs are not stored)
+    const int r = 8 * j + r8;
+    const int row = SWIGLU ? min(it.f0 + 32 * wv + (r & 31), a.N - 1) + (r >> 5) * upoff
+                           : min(it.f0 + 64 * wv + r, a.N - 1);
+    s.w[j] = wbase + (int64_t)row * wld + ((lane & 7) ^ ((r8 & 3) | ((j & 1) << 2))) * 8;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {  // tokens past the tile: its first one
+    const int r = 8 * (4 * j + wv) + r8;
+    const int slot = it.t0 + (r < it.count ? r : 0);
+    if (it.shared) s.t[j] = a.X2 + it.g * a.x2g + (int64_t)slot * a.x2s + pc;
+    else s.t[j] = a.X + it.g * a.xg + (int64_t)(a.slot_row ? a.slot_row[slot] / a.slot_div : slot) * a.xs + pc;
+  }
+}
+
+__device__ __forceinline__ void big_load(const bf16_t* src, uint8_t* dst) {
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+__device__ __forceinline__ void big_wload(const BigSrc& s, uint8_t* lds, int j, int chunk, int stage) {
+  big_load(s.w[j] + chunk * 64, lds + stage * kBigStage + (64 * (threadIdx.x >> 6) + 8 * j) * 128);
+}
+__device__ __forceinline__ void big_tload(const BigSrc& s, uint8_t* lds, int j, int chunk, int stage) {
+  big_load(s.t[j] + chunk * 64, lds + stage * kBigStage + (kBigRows + 8 * (4 * j + (threadIdx.x >> 6))) * 128);
+}
+
+// The accumulators stay in the 256 AGPRs of a lone wave per SIMD (as a builtin the compiler copies
+// them to and from VGPRs between the MFMAs, and spills).  The hazards the compiler would cover are
+// met by hand: nothing but these MFMAs touches an accumulator between the two s_nop fences.
+__device__ __forceinline__ void mfma_acc(floatx4_t& c, const bf16x8_t& a, const bf16x8_t& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void acc_fence() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15"); }
+__device__ __forceinline__ float acc_read(float c) {
+  float f;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(f) : "a"(c));
+  return f;
+}
+__device__ __forceinline__ void big_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// One item of NG x 64 tokens whose chunks 0 and 1 are in (or on their way to) the stages; on
+// return chunks 0 and 1 of the workgroup's next item jn are.
+template <bool SWIGLU, int NG>
+__device__ __forceinline__ void big_tile(const GemmArgs& a, const BigShape& sh, uint8_t* lds, BigItem& item,
+                                         BigSrc& src, int jn, bool more) {
+  constexpr int RB = 128;
+  constexpr int LT = 2 * NG;            // token ring loads per wave per chunk
+  constexpr int XM = 4, XN = 4 * NG;    // MFMA blocks per wave: 64 weight rows x 64 NG tokens
+  constexpr int XL = XN - 4;            // token blocks before the last four
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, kg = lane >> 4;
+  const int nch = a.K / 64, odd = nch & 1;
+  floatx4_t acc[XM][XN];
+#pragma unroll
+  for (int x = 0; x < XM; ++x)
+#pragma unroll
+    for (int y = 0; y < XN; ++y) acc[x][y] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  bf16x8_t af[2][4], bfr[XL > 0 ? XL : 1], hi[2][4];
+  // weight fragment x takes the wave's rows 8 (li / 4) + 4 xr + li % 4 of a 32-row half
+  const int arow = (64 * wv + 8 * (li >> 2) + (li & 3)) * RB, brow = (kBigRows + li) * RB;
+  const int sw0 = (kg ^ (li & 7)) * 16, sw1 = ((4 + kg) ^ (li & 7)) * 16;
+  auto reada = [&](int st, int s, int x) {
+    const int half = SWIGLU ? x & 1 : x >> 1, xr = SWIGLU ? x >> 1 : x & 1;
+    return *reinterpret_cast<const bf16x8_t*>(lds + st * kBigStage + arow + (32 * half + 4 * xr) * RB + (s ? sw1 : sw0));
+  };
+  auto readb = [&](int st, int s, int y) {
+    return *reinterpret_cast<const bf16x8_t*>(lds + st * kBigStage + brow + y * 16 * RB + (s ? sw1 : sw0));
+  };
+  // K half s of the chunk in stage i: its fragments are in af[s], bfr and hi[s]; the next half's
+  // replace them, each right after its last use (the last four token blocks have a second set, so
+  // that no read is issued within 15 MFMAs of the wait before the barrier).  At most one other
+  // instruction between two MFMAs (16 cycles each, 4 of them to issue): a burst of them leaves
+  // the matrix core idle.
+  auto half = [&](auto stage, auto sub, auto&& extra) {
+    constexpr int i = decltype(stage)::value, s = decltype(sub)::value;
+    constexpr int ni = s ? i ^ 1 : i, ns = s ^ 1;  // the fragments read now: stage, K half
+#pragma unroll
+    for (int y = 0; y < XN; ++y)
+#pragma unroll
+      for (int x = 0; x < XM; ++x) {
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_acc(acc[x][y], af[s][x], y < XL ? bfr[y < XL ? y : 0] : hi[s][y < XL ? 0 : y - XL]);
+        if (XN == 4) {
+          if (y < 2) {
+            if (x < 2) af[ns][2 * y + x] = reada(ni, ns, 2 * y + x);
+            else hi[ns][2 * y + x - 2] = readb(ni, ns, 2 * y + x - 2);
+          }
+        } else {
+          if (x == 0 && y >= 1 && y <= XL) bfr[y - 1] = readb(ni, ns, y - 1);
+          if (x == 1 && y < 4) af[ns][y] = reada(ni, ns, y);
+          if (x == 2 && y < 4) hi[ns][y] = readb(ni, ns, XL + y);
+        }
+        extra(4 * y + x);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // cc: the chunk to request into stage i once every wave has read it
+  auto step = [&](auto stage, int cc) {
+    constexpr int i = decltype(stage)::value;
+    half(stage, Int<0>{}, [](int) {});
+    // this wave's reads of stage i are done and its loads of the other stage's chunk have
+    // landed, then every wave's
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    big_barrier();
+    half(stage, Int<1>{}, [&](int u) {  // ring load q after MFMA u
+      constexpr int NL = 8 + LT, per = 4 * XN / NL;
+#pragma unroll
+      for (int q = 0; q < NL; ++q)
+        if (u == q * per + (XN == 4 ? 0 : 3)) {
+          if (q < 8) big_wload(src, lds, q, cc, i);
+          else big_tload(src, lds, q - 8, cc, i);
+        }
+    });
+  };
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  acc_fence();
+  big_barrier();
+#pragma unroll
+  for (int x = 0; x < XM; ++x) af[0][x] = reada(0, 0, x);
+#pragma unroll
+  for (int y = 0; y < XL; ++y) bfr[y] = readb(0, 0, y);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) hi[0][k] = readb(0, 0, XL + k);
+  BigItem next = item;
+  int c = 0;
+  do {
+    int c0 = c + 2 - odd, c1 = c + 3 - odd;
+    c += 2;
+    if (c >= nch) {  // the last pair requests the next item's first chunks (none: this one's again)
+      if (more) {
+        next = big_item<SWIGLU>(a, sh, jn);
+        big_src<SWIGLU>(a, next, src);
+      }
+      c0 = 0;
+      c1 = min(1, nch - 1);
+    }
+    step(Int<0>{}, c0);
+    step(Int<1>{}, c1);
+  } while (c < nch);
+  acc_fence();
+  // the next item's token rows that this tile's loads did not cover
+  if (NG < 4 && more && next.count > 64 * NG) {
+    big_barrier();
+    const int c1 = min(1, nch - 1);
+#pragma unroll
+    for (int j = LT; j < 8; ++j) {
+      big_tload(src, lds, j, 0, 0);
+      big_tload(src, lds, j, c1, 1);
+    }
+  }
+  // lane (li, kg) holds, for token 16y + li, features 8 kg .. 8 kg + 7 of each of the wave's
+  // output blocks of 32 (block o: plain fragments 2o and 2o + 1; SwiGLU: gate fragments 0 and 2,
+  // up 1 and 3)
+  constexpr int XO = SWIGLU ? 1 : 2;
+  const int n0 = item.f0 + (SWIGLU ? 32 : 64) * wv + 8 * kg;
+  {
+    const bool shared = item.shared, f32 = shared ? !SWIGLU : a.out_f32, exact = shared || a.exact_f32;
+    const int64_t ys = shared ? a.y2s : a.ys;
+    char* const yb = reinterpret_cast<char*>(shared ? a.Y2 : a.Y) +
+                     (item.g * (shared ? a.y2g : a.yg) + item.t0 * ys + n0) * (f32 ? 4 : 2);
+    const bf16_t* const rb = a.res && !shared ? a.res + item.t0 * a.rs + n0 : nullptr;
+#pragma unroll
+    for (int y = 0; y < XN; ++y) {
+      const int t = 16 * y + li;
+      if (t >= item.count) continue;
+#pragma unroll
+      for (int o = 0; o < XO; ++o) {
+        if (n0 + 32 * o >= a.N) break;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (SWIGLU) v[e] = swiglu_bf(acc_read(acc[2 * (e >> 2)][y][e & 3]), acc_read(acc[2 * (e >> 2) + 1][y][e & 3]));
+          else v[e] = acc_read(acc[2 * o + (e >> 2)][y][e & 3]);
+        }
+        if (rb) {
+          const bf16_t* const rp = rb + (int64_t)t * a.rs + 32 * o;
+          float r[8];
+          if (sh.wide) {
+            unpack8(ldg16(rp), r);
+          } else {
+            const uint2 r0 = reinterpret_cast<const uint2*>(rp)[0], r1 = reinterpret_cast<const uint2*>(rp)[1];
+            unpack8(make_uint4(r0.x, r0.y, r1.x, r1.y), r);
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = r[e] + rbf(v[e]);
+        }
+        const int64_t off = (int64_t)t * ys + 32 * o;
+        if (f32) {
+          if (!exact) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = rbf(v[e]);
+          }
+          float4* p = reinterpret_cast<float4*>(yb + off * 4);
+          p[0] = make_float4(v[0], v[1], v[2], v[3]);
+          p[1] = make_float4(v[4], v[5], v[6], v[7]);
+        } else {
+          const uint4 w = pack8(v);
+          if (sh.wide) {
+            *reinterpret_cast<uint4*>(yb + off * 2) = w;
+          } else {
+            reinterpret_cast<uint2*>(yb + off * 2)[0] = make_uint2(w.x, w.y);
+            reinterpret_cast<uint2*>(yb + off * 2)[1] = make_uint2(w.z, w.w);
+          }
+        }
+      }
+    }
+  }
+  item = next;
+}
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_big_kernel(const GemmArgs a, const BigShape sh) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int items = big_items(a, sh), per = (items + 7) / 8;
+  const int lo = (blockIdx.x % 8) * per, end = min(lo + per, items), stride = gridDim.x / 8;
+  int j = lo + blockIdx.x / 8;
+  if (j >= end) return;
+  BigItem item = big_item<SWIGLU>(a, sh, j);
+  BigSrc src;
+  big_src<SWIGLU>(a, item, src);
+  const int nch = a.K / 64;
+  if (nch & 1) {  // a chunk of zeros first, so that chunks come in pairs (one item per workgroup then)
+    const u32x4_t z = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < kBigStage / 4096; ++i)
+      *reinterpret_cast<u32x4_t*>(lds + (256 * i + (int)threadIdx.x) * 16) = z;
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) big_wload(src, lds, q, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (32 * q < item.count) big_tload(src, lds, q, 0, 0);
+  }
+  const int c1 = nch & 1 ? 0 : 1;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) big_wload(src, lds, q, c1, 1);
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (32 * q < item.count) big_tload(src, lds, q, c1, 1);
+  for (;; j += stride) {
+    const int jn = j + stride;
+    const bool more = jn < end;
+    if (item.count <= 64) big_tile<SWIGLU, 1>(a, sh, lds, item, src, jn, more);
+    else if (item.count <= 128) big_tile<SWIGLU, 2>(a, sh, lds, item, src, jn, more);
+    else if (item.count <= 192) big_tile<SWIGLU, 3>(a, sh, lds, item, src, jn, more);
+    else big_tile<SWIGLU, 4>(a, sh, lds, item, src, jn, more);
+    if (!more) break;
+  }
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // the repeats land before the LDS is released
+}
+
+// grouped: max_tiles entries of a table of tiles of up to 256 tokens; dense: a.rows tokens in
+// tiles of 64 ng
+static void launch_big(const GemmArgs& a, bool swiglu, hipStream_t st, int ng, int max_tiles = 0) {
+  BigShape sh;
+  sh.tokens = 64 * ng;
+  sh.nfb = swiglu ? (a.N + kBigRows / 2 - 1) / (kBigRows / 2) : (a.N + kBigRows - 1) / kBigRows;
+  sh.tiles = a.tiles ? max_tiles : (a.rows + sh.tokens - 1) / sh.tokens;
+  sh.wide = dsv2_aligned16(a.Y) && a.ys % 8 == 0 && a.yg % 8 == 0 && a.N % 8 == 0 &&
+            (!a.res || (dsv2_aligned16(a.res) && a.rs % 8 == 0)) &&
+            (!a.Y2 || (dsv2_aligned16(a.Y2) && a.y2s % 8 == 0 && a.y2g % 8 == 0));
+  const int64_t items = ((int64_t)sh.tiles + (a.W2 ? 2 * a.s_tiles : 0)) * sh.nfb;
+  const int64_t all = (items + 7) / 8 * 8;
+  // an odd number of K chunks starts with a chunk of zeros, which only a workgroup's first item has
+  const int nwg = (int)((a.K / 64) & 1 ? all : (all < kBigWgs ? all : (int64_t)kBigWgs));
+  if (swiglu) hipLaunchKernelGGL(gemm_big_kernel<true>, dim3(nwg), dim3(256), 2 * kBigStage, st, a, sh);
+  else hipLaunchKernelGGL(gemm_big_kernel<false>, dim3(nwg), dim3(256), 2 * kBigStage, st, a, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -1226,45 +1513,66 @@ static int launch_gemm(const GemmArgs& a, int tb, bool swiglu, int grid_y, hipSt
 
 static int pick_tb(int rows) { return rows <= 16 ? 1 : (rows <= 32 ? 2 : (rows <= 64 ? 4 : 8)); }
 
+// Which direct-to-LDS shape a dense GEMM takes: 0 the 64 x 64 ring (gemm_dma_kernel), 1..4 the
+// 256 x 64 n tiles of gemm_big_kernel, -1 neither (the shapes below).
+// From 65 rows the ring beats them where it has enough items: SwiGLU from 128 (MI355X, 2816
+// features x 2048: 128 rows 20.0 -> 11.3 us; 10944: 42 -> 24.6), many features (3648: 13.8 ->
+// 11.6) and else 160 (2048 x 2048: 211 rows, 128 items, 10.4 against 11.5 us; 300 rows, 160
+// items, 14.8 -> 11.6; K = 10944: 300 rows 61 -> 42); the lm_head (102400 x 2048) and the dense
+// layer's gate_up (SwiGLU, 10944 x 2048) from 33 rows (64 rows: 116 -> 100 and 35.6 -> 28.8).
+// Ring or large tiles: the cheaper by their measured times (us; K = 2048, 2816, 10944 at 512 to
+// 8192 rows, within about 15% of each).  The ring takes 4 + 0.034 per item and 2048 of K (512
+// items resident); the large tiles 8 + per round of 256 items K / 64 chunks of 0.75 / 0.82 / 0.95
+// / 1.2 us for 64 / 128 / 192 / 256 tokens and 3 between rounds.  E.g. 1149 rows x 2048 x 2048:
+// ring 24.8, large 29.8 / 33.6 / 38.8 / 47.2; 2300 rows x 3648: 73 against 77 / 62 / 42 / 50;
+// 8192 rows x 10944 (SwiGLU): 1525 against 637 with 256 tokens; lm_head at 200 rows 199 -> 141.
+static int dense_tiles(int rows, int N, int K, bool swiglu) {
+  if (swiglu ? N % 32 != 0 : N % 64 != 0) return -1;
+  const int64_t items = (int64_t)((rows + 63) / 64) * (swiglu ? N / 32 : N / 64);
+  const bool wide = rows > 32 && N >= (swiglu ? 8192 : 16384);
+  if (!wide && (rows <= 64 || items < (swiglu ? 128 : (N >= 3072 ? 100 : 160)))) return -1;
+  const double ring_us = 4.0 + K / 2048.0 * (0.034 * items > 8.0 ? 0.034 * items : 8.0);
+  const double chunk_us[4] = {0.75, 0.82, 0.95, 1.2};
+  int best = 0;
+  double best_us = ring_us;
+  const int rows_wg = swiglu ? kBigRows / 2 : kBigRows;
+  for (int ng = 1; ng <= 4; ++ng) {
+    const int64_t n = (int64_t)((rows + 64 * ng - 1) / (64 * ng)) * ((N + rows_wg - 1) / rows_wg);
+    const double us = 5.0 + (double)((n + kBigWgs - 1) / kBigWgs) * (3.0 + K / 64 * chunk_us[ng - 1]);
+    if (us < best_us) {
+      best_us = us;
+      best = ng;
+    }
+  }
+  return best;
+}
+
 // Dense (implicit-tile) shapes whose row blocks alone cannot fill the chip, measured on
 // MI355X at 16..256 tokens: the one-shot kernel for short K and up to 64 tokens; the
-// token-rows-in-LDS kernel (64-row workgroups sharing token chunks) for more tokens, with
+// token-rows-in-LDS kernel (64-row workgroups sharing token chunks) for more, with
 // the largest token tile that still gives ~200 workgroups (SwiGLU: 64-token tiles); long K
 // with few features on 16/32-token tiles.  Returns false (nothing launched) for shapes left
 // to launch_gemm: huge N, long K with SwiGLU or groups, or N not a multiple of 16*rbw.
-constexpr int kBigTileRows = 512;
 static bool launch_dense_os(GemmArgs a, int groups, bool swiglu, hipStream_t st) {
   const int rows = a.rows, K = a.K;
+  const int ring = groups == 1 ? dense_tiles(rows, a.N, K, swiglu) : -1;
+  if (ring > 0) {
+    launch_big(a, swiglu, st, ring);
+    return true;
+  }
+  if (ring == 0) {
+    launch_dma(a, swiglu, st);
+    return true;
+  }
   if (K > 4096 && !swiglu && groups == 1 && a.N % 64 == 0 && a.N < 16384) {
     // long K, few features (dense layer-0 down, K = 10944): token-rows-in-LDS tiles of 16 /
-    // 32 tokens with row-contiguous weight staging (bsz=256: 51 us vs 97 us for the k-split
-    // kernel's MFMA-fragment-order loads; bsz=64: 41 vs 62 us)
+    // 32 tokens with row-contiguous weight staging (bsz=64: 41 vs 62 us for the k-split
+    // kernel's MFMA-fragment-order loads)
     const int tb = rows <= 64 ? 1 : 2;
     a.tiles_per_group = (rows + 16 * tb - 1) / (16 * tb);
     if (a.tiles_per_group > 65535) return false;
     if (tb == 1) launch_xlds_variant<1, false, 4, true, 2>(a, a.tiles_per_group, st);
     else launch_xlds_variant<2, false, 4, true, 2>(a, a.tiles_per_group, st);
-    return true;
-  }
-  if (groups == 1 && K <= 4096 && rows >= kBigTileRows && a.N >= kBigRows &&
-      a.N % (swiglu ? kBigRows / 2 : 64) == 0) {
-    // prefill-size row counts: 128 weight rows x 128 tokens per workgroup
-    launch_dma(a, swiglu, st, 0, true);
-    return true;
-  }
-  if (!swiglu && groups == 1 && K <= 4096 && a.N % 64 == 0 &&
-      ((rows > 128 && (a.N / 64) * ((rows + 63) / 64) >= 192) || (rows > 32 && a.N >= 16384))) {
-    // direct-to-LDS ring: 128+ tokens with enough 64 x 64 tiles to fill the chip (qkv_a at
-    // 256 tokens, 228 workgroups: 12.9 vs 16.1 us in the decode step; N = 2048 gives only 128
-    // and stays on the token-rows-in-LDS shape's 32-token tiles, o_proj 12.9 vs 14.0 us), and
-    // the lm_head (N = 102400) from 33 tokens (64: 104 vs 121 us; 256: 251 vs 301 us)
-    launch_dma(a, false, st);
-    return true;
-  }
-  if (swiglu && groups == 1 && K <= 4096 && a.N % 32 == 0 && rows > 128) {
-    // SwiGLU on the ring (32 features x 64 tokens per workgroup): shared experts and the dense
-    // layer-0 gate_up above 128 tokens (reference workload at 256 rows 39.3k -> 39.4k tok/s)
-    launch_dma(a, true, st);
     return true;
   }
   if (K > 4096 || (int64_t)a.N * groups >= 16384) return false;
@@ -1446,7 +1754,8 @@ extern "C" int dsv2_moe_grouped_gateup(const void* xn, const int32_t* sorted_rou
   if ((tile_tokens == 64 && inter % 32 == 0) || (tile_tokens == kBigTokens && inter % (kBigRows / 2) == 0)) {
     // 64- and 256-token tiles on the direct-to-LDS ring (reference workload, 6 experts x 256
     // tokens: 45 us vs 71 us for the token-rows-in-LDS shape; x 64 tokens: 26.0 vs 26.8 us)
-    launch_dma(a, true, (hipStream_t)stream, max_tiles, tile_tokens == kBigTokens);
+    if (tile_tokens == kBigTokens) launch_big(a, true, (hipStream_t)stream, 4, max_tiles);
+    else launch_dma(a, true, (hipStream_t)stream, max_tiles);
     return dsv2_launch_status("moe_grouped_gateup");
   }
   DSV2_REQUIRE(tile_tokens != kBigTokens, DSV2_E_SHAPE, "moe_grouped_gateup: 256-token tiles need inter %% %d", kBigRows / 2);
@@ -1492,7 +1801,8 @@ extern "C" int dsv2_moe_grouped_gateup_shared(const void* xn, int rows, const in
   a.y2s = 2 * inter;
   a.y2g = inter;
   if (tile_tokens >= 64) {
-    launch_dma(a, true, (hipStream_t)stream, max_tiles, tile_tokens == kBigTokens);
+    if (tile_tokens == kBigTokens) launch_big(a, true, (hipStream_t)stream, 4, max_tiles);
+    else launch_dma(a, true, (hipStream_t)stream, max_tiles);
     return dsv2_launch_status("moe_grouped_gateup_shared");
   }
   return launch_gemm(a, tile_tb(tile_tokens), true, 2 * a.s_tiles + max_tiles, (hipStream_t)stream);
@@ -1537,7 +1847,8 @@ extern "C" int dsv2_moe_grouped_down_shared(const void* hsorted, int rows, const
   a.y2s = 2048;
   a.y2g = (int64_t)rows * 2048;
   if (tile_tokens >= 64) {
-    launch_dma(a, false, (hipStream_t)stream, max_tiles, tile_tokens == kBigTokens);
+    if (tile_tokens == kBigTokens) launch_big(a, false, (hipStream_t)stream, 4, max_tiles);
+    else launch_dma(a, false, (hipStream_t)stream, max_tiles);
     return dsv2_launch_status("moe_grouped_down_shared");
   }
   return launch_gemm(a, tile_tb(tile_tokens), false, 2 * a.s_tiles + max_tiles, (hipStream_t)stream);
@@ -1570,7 +1881,8 @@ extern "C" int dsv2_moe_grouped_down(const void* hsorted, const int32_t* tiles, 
   a.yg = 0;
   if (tile_tokens >= 64) {
     // 6 experts x 256 tokens: 24 us vs 35 us; x 64 tokens: 12.0 vs 16.3 us
-    launch_dma(a, false, (hipStream_t)stream, max_tiles, tile_tokens == kBigTokens);
+    if (tile_tokens == kBigTokens) launch_big(a, false, (hipStream_t)stream, 4, max_tiles);
+    else launch_dma(a, false, (hipStream_t)stream, max_tiles);
     return dsv2_launch_status("moe_grouped_down");
   }
   return launch_gemm(a, tile_tb(tile_tokens), false, max_tiles, (hipStream_t)stream);

@@ -1142,3 +1142,66 @@ def test_stream_copy_exact(nbytes):
     torch.cuda.synchronize()
     assert torch.equal(dst[:nbytes], src)
     assert torch.all(dst[nbytes:] == 7)
+
+
+@pytest.mark.parametrize("rows,K,N,swiglu,out", [
+    (2300, 704, 3648, False, "bf16"),      # odd K chunks, a ragged last feature block, 192-token tiles
+    (2300, 704, 3648, False, "residual"),
+    (2300, 704, 3648, False, "narrow"),    # 8-byte aligned output and residual rows
+    (4100, 192, 2080, True, "bf16"),       # SwiGLU, the last block a quarter full, 3 K chunks
+    (8129, 64, 4096, False, "f32"),        # one K chunk, several items per workgroup
+    (5000, 128, 2048, False, "exact"),
+])
+def test_large_tile_gemm_edges(rows, K, N, swiglu, out):
+    """Shapes whose cost picks the 256-row tiles, against fp32 torch: one bf16 round of an fp32 sum
+    is 2^-9 of the value (4e-3 of the largest bounds it), with a residual there are two (the sum,
+    then sum + residual: 8e-3), with SwiGLU four (1e-2)."""
+    x, w = rnd(rows, K, seed=90), rnd((2 if swiglu else 1) * N, K, seed=91, std=K ** -0.5)
+    ld = N + 4 if out == "narrow" else N
+    flags = {"f32": 2, "exact": 4}.get(out, 0) | (1 if swiglu else 0)
+    y = torch.empty(rows, ld, device=DEV, dtype=torch.float32 if flags & 6 else BF)
+    res = rnd(rows, ld, seed=92) if out in ("residual", "narrow") else None
+    call("dsv2_gemm_bf16", x.data_ptr(), K, 0, rows, K, w.data_ptr(), 0, N, 1, None if res is None else res.data_ptr(),
+         ld, y.data_ptr(), ld, 0, flags, st())
+    ref = x.float() @ w.float().t()
+    if swiglu:
+        ref = torch.nn.functional.silu(ref[:, :N]) * ref[:, N:]
+    if res is not None:
+        ref = ref + res[:, :N].float()
+    assert rel_err(y[:, :N].float(), ref) < {"exact": 1e-5}.get(out, 1e-2 if swiglu else (8e-3 if res is not None else 4e-3))
+
+
+@pytest.mark.parametrize("inter", [128, 192])
+def test_grouped_large_tile_token_counts(inter):
+    """256-token expert tiles holding 1 to 256 tokens (each of the kernel's token loops and its
+    edges) against the same routes on 64-token tiles: the gate_up and down products are the same
+    fp32 sums in another order, rounded to bf16 (one ulp, 2^-7 of the value, where they straddle a
+    rounding boundary)."""
+    counts = [1, 16, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 512, 700] + [0] * 40 + [33] * 8
+    routes = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(counts)])
+    tokens = -(-routes.numel() // 6)
+    ids = torch.zeros(tokens * 6, dtype=torch.int32)
+    ids[:routes.numel()] = routes[torch.randperm(routes.numel(), generator=torch.Generator().manual_seed(1))]
+    ids = ids.to(DEV)
+    R = tokens * 6
+    x = rnd(tokens, 2048, seed=93)
+    gu, dn = rnd(64, 2 * inter, 2048, seed=94, std=0.02), rnd(64, 2048, inter, seed=95, std=0.1)
+    got = {}
+    for tile in (64, 256):
+        n = -(-R // tile) + 64
+        i32 = lambda *s: torch.empty(*s, dtype=torch.int32, device=DEV)  # noqa: E731
+        srt, pos, tiles, nt = i32(R), i32(R), i32(n, 4), i32(1)
+        call("dsv2_moe_bucket", ids.data_ptr(), tokens, tile, srt.data_ptr(), pos.data_ptr(), tiles.data_ptr(),
+             nt.data_ptr(), st())
+        hs, ys = torch.empty(R, inter, dtype=BF, device=DEV), torch.empty(R, 2048, dtype=BF, device=DEV)
+        if inter % 128 == 0 or tile == 64:
+            call("dsv2_moe_grouped_gateup", x.data_ptr(), srt.data_ptr(), tiles.data_ptr(), nt.data_ptr(), n, tile,
+                 gu.data_ptr(), inter, hs.data_ptr(), st())
+        else:
+            hs = got[64][0]  # 256-token gate_up tiles need inter % 128: only the down (odd K chunks)
+        call("dsv2_moe_grouped_down", (got[64][0] if tile == 256 else hs).data_ptr(), tiles.data_ptr(), nt.data_ptr(), n,
+             tile, dn.data_ptr(), inter, ys.data_ptr(), st())
+        got[tile] = (hs, ys)
+    for a, b in zip(got[256], got[64]):
+        assert rel_err(a.float(), b.float()) < 2 ** -7
+        assert (a == b).float().mean() > 0.9
