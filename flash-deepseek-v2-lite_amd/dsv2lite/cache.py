@@ -48,6 +48,7 @@ class CompressedKVCache:
         for b, c in enumerate(self.capacities):
             bases.append(start + (((7 * b) % STAGGER_PHASES) * STAGGER_TILE if stagger else 0))
             start += c + pad
+        self.bases = bases  # host copy of `base`
         self.total = start
         self.row = row
         self.data = torch.zeros(n_layers, self.total, row, dtype=torch.bfloat16, device=device)

@@ -103,33 +103,67 @@ class PrefillPlan:
         self.kexp, self.vexp = kexp, vexp
 
 
-def _segments(seq: torch.Tensor) -> list[tuple[int, int, int]]:
-    """(first chunk row, rows, sequence) of each run of one sequence's rows in a chunk."""
+def _segments(seq: torch.Tensor, posv: torch.Tensor) -> list[tuple[int, int, int, int]]:
+    """(first chunk row, rows, sequence, first position) of each run of one sequence's rows in a
+    chunk."""
     vals, counts = torch.unique_consecutive(seq, return_counts=True)
     out, r = [], 0
     for s, cnt in zip(vals.tolist(), counts.tolist()):
-        out.append((r, cnt, s))
+        out.append((r, cnt, s, int(posv[r])))
         r += cnt
     return out
 
 
-def _group_tiles(segs, posv: torch.Tensor, bases: list[int], tile: int) -> tuple[torch.Tensor, int, int]:
+def _chunk_segments(lens: list[int], s: int, e: int) -> list[tuple[int, int, int, int]]:
+    """_segments of rows [s, e) of prompts of the given lengths laid one after the other."""
+    out, start = [], 0
+    for j, n in enumerate(lens):
+        lo, hi = max(s, start), min(e, start + n)
+        if lo < hi:
+            out.append((lo - s, hi - lo, j, lo - start))
+        start += n
+    return out
+
+
+def _group_tiles(segs, bases: list[int], tile: int) -> tuple[list[tuple[int, int, int, int]], int, int]:
     out, lo, hi = [], None, None
-    for r, cnt, s in segs:
-        p_first = int(posv[r])
+    for r, cnt, s, p_first in segs:
         for a in range(0, cnt, tile):
             out.append((r + a, min(tile, cnt - a), p_first + a, bases[s]))
         lo = bases[s] if lo is None else min(lo, bases[s])
         last = bases[s] + p_first + cnt
         hi = last if hi is None else max(hi, last)
-    return torch.tensor(out, dtype=torch.int32).reshape(-1, 4), int(lo), int(hi - lo)
+    return out, int(lo), int(hi - lo)
+
+
+def _plan_groups(segs, bases: list[int], tile: int = 128,
+                 slack: int = 4096) -> list[tuple[list[tuple[int, int, int, int]], int, int]]:
+    groups, cur, lo, hi, used = [], [], 0, 0, 0
+    for seg in segs:
+        _, cnt, s, p_first = seg
+        need = p_first + cnt
+        a, e = bases[s], bases[s] + need
+        if cur and max(hi, e) - min(lo, a) <= 2 * (used + need) + slack:
+            cur.append(seg)
+            lo, hi, used = min(lo, a), max(hi, e), used + need
+            continue
+        if cur:
+            groups.append(cur)
+        cur, lo, hi, used = [seg], a, e, need
+    groups.append(cur)
+    return [_group_tiles(g, bases, tile) for g in groups]
+
+
+def _tile_tensor(tiles: list[tuple[int, int, int, int]]) -> torch.Tensor:
+    return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 4)
 
 
 def prefill_tiles(seq: torch.Tensor, posv: torch.Tensor, bases: list[int], tile: int = 128) -> tuple[torch.Tensor, int, int]:
     """Query tiles of one chunk (seq[r]: sequence of chunk row r, posv[r]: its position;
     rows of a sequence are consecutive with consecutive positions) and the cache row range
     its attention reads: from the lowest sequence base to the last position of any row."""
-    return _group_tiles(_segments(seq), posv, bases, tile)
+    t, lo, n = _group_tiles(_segments(seq, posv), bases, tile)
+    return _tile_tensor(t), lo, n
 
 
 def prefill_groups(seq: torch.Tensor, posv: torch.Tensor, bases: list[int], tile: int = 128,
@@ -138,19 +172,35 @@ def prefill_groups(seq: torch.Tensor, posv: torch.Tensor, bases: list[int], tile
     twice the rows they attend (plus `slack`): with slots far apart (capacities much larger
     than the prompts) one range over the whole chunk would expand every slot's unused
     capacity in between.  Each group: (tiles, exp_lo, exp_rows)."""
-    groups, cur, lo, hi, used = [], [], 0, 0, 0
-    for r, cnt, s in _segments(seq):
-        need = int(posv[r]) + cnt
-        a, e = bases[s], bases[s] + need
-        if cur and max(hi, e) - min(lo, a) <= 2 * (used + need) + slack:
-            cur.append((r, cnt, s))
-            lo, hi, used = min(lo, a), max(hi, e), used + need
-            continue
-        if cur:
-            groups.append(cur)
-        cur, lo, hi, used = [(r, cnt, s)], a, e, need
-    groups.append(cur)
-    return [_group_tiles(g, posv, bases, tile) for g in groups]
+    return [(_tile_tensor(t), lo, n) for t, lo, n in _plan_groups(_segments(seq, posv), bases, tile, slack)]
+
+
+class _Upload:
+    """Host tensors gathered into one pinned buffer and one asynchronous copy.  A prefill's ids,
+    positions, cache bases and tile tables as separate copies from pageable memory each waited for
+    the stream's earlier work (MI355X, four layers: insert of 211 tokens 1555 -> 1364 us, prefill of
+    9,341 tokens in two chunks 10.6 -> 9.7 ms)."""
+
+    def __init__(self) -> None:
+        self.parts: list[torch.Tensor] = []
+        self.size = 0
+
+    def add(self, t: torch.Tensor) -> int:
+        self.parts.append(t.contiguous())
+        self.size += -(-t.numel() * t.element_size() // 16) * 16
+        return len(self.parts) - 1
+
+    def send(self, device) -> list[torch.Tensor]:
+        """The parts on `device`, in the order they were added."""
+        host = torch.empty(max(self.size, 16), dtype=torch.uint8, pin_memory=True)
+        at, offs = 0, []
+        for t in self.parts:
+            n = t.numel() * t.element_size()
+            host[at:at + n].copy_(t.reshape(-1).view(torch.uint8))
+            offs.append((at, n))
+            at += -(-n // 16) * 16
+        dev = host.to(device, non_blocking=True)
+        return [dev[o:o + n].view(t.dtype).reshape(t.shape) for (o, n), t in zip(offs, self.parts)]
 
 
 class RowBuffers:
@@ -595,18 +645,34 @@ class DecodeEngine:
                 raise ValueError(f"prompt of length {n} does not fit slot {b} (capacity {self.cache.capacities[b]})")
         dev = self.device
         k = len(slots)
-        seq = torch.cat([torch.full((n,), j, dtype=torch.int64) for j, n in enumerate(lens)])  # prompt index
-        slot_t = torch.tensor(slots, dtype=torch.int64)
-        posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
-        ids_all = torch.cat([p.reshape(-1).to(torch.int64).cpu() for p in prompts])
-        base_all = self.cache.base.cpu()[slot_t[seq]]
-        cap_all = self.cache.cap.cpu()[slot_t[seq]]
-        total = seq.numel()
+        total = sum(lens)
         max_rows = min(self.max_prefill_rows, total)
+        bases = [self.cache.bases[b] for b in slots]
+        # everything the chunks read, planned here and sent in one copy
+        up = _Upload()
+        on_host = all(p.device.type == "cpu" for p in prompts)
+        if on_host:
+            i_ids = up.add(torch.cat([p.reshape(-1).to(torch.int64) for p in prompts]))
+        counts = torch.tensor(lens)
+        i_pos = up.add(torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]))
+        i_base = up.add(torch.repeat_interleave(torch.tensor(bases, dtype=torch.int64), counts))
+        i_cap = up.add(torch.repeat_interleave(
+            torch.tensor([self.cache.capacities[b] for b in slots], dtype=torch.int32), counts))
+        i_slot = up.add(torch.tensor(slots, dtype=torch.int64))
+        i_lens = up.add(counts.to(torch.int32))
+        chunks = []
+        for s in range(0, total, max_rows):
+            e = min(total, s + max_rows)
+            segs = _chunk_segments(lens, s, e)
+            groups = [(up.add(_tile_tensor(t)), lo, n) for t, lo, n in _plan_groups(segs, bases)]
+            last = [(r + cnt - 1, j) for r, cnt, j, p in segs if p + cnt == lens[j]]  # (chunk row, prompt)
+            rw = up.add(torch.tensor(last, dtype=torch.int64).reshape(-1, 2).t())
+            chunks.append((s, e, groups, rw, len(last)))
+        sent = up.send(dev)
+        ids_all = sent[i_ids] if on_host else torch.cat([p.reshape(-1).to(dev, torch.int64) for p in prompts])
+        pos_all, base_all, cap_all, slot_d = sent[i_pos], sent[i_base], sent[i_cap], sent[i_slot]
         pb = RowBuffers(self.cfg, max_rows, "batch", self.max_pos, dev, prefill=True)
-        bases = [int(x) for x in self.cache.base.cpu()[slot_t]]
-        plans = [prefill_groups(seq[s:s + max_rows], posv[s:s + max_rows], bases) for s in range(0, total, max_rows)]
-        n_exp = max(g[2] for p in plans for g in p)
+        n_exp = max(g[2] for c in chunks for g in c[2])
         nh, dk = self.cfg.n_heads, self.cfg.qk_nope
         kexp = torch.empty(n_exp, nh, dk, dtype=BF16, device=dev)
         vexp = torch.empty(n_exp, nh, self.cfg.v_dim, dtype=BF16, device=dev)
@@ -614,27 +680,19 @@ class DecodeEngine:
         last_xn = torch.empty_like(last_h)
         st = _hip.stream_ptr(dev)
         acc: dict = {}
-        for s in range(0, total, max_rows):
-            e = min(total, s + max_rows)
+        for s, e, groups, rw, n_last in chunks:
             R = e - s
-            ids_c = ids_all[s:e].to(dev)
-            pos_c = posv[s:e].to(dev)
-            base_c = base_all[s:e].to(dev)
-            cap_c = cap_all[s:e].to(dev)
-            is_last = (posv[s:e] + 1) == torch.tensor(lens)[seq[s:e]]
-            rows = torch.nonzero(is_last).flatten()
-            rows_d = rows.to(dev)
-            which = seq[s:e][rows].to(dev)
+            rows_d, which = sent[rw][0], sent[rw][1]
             crec = [] if record is not None else None
-            pf = PrefillPlan([(t.to(dev), lo, n) for t, lo, n in plans[s // max_rows]], kexp, vexp)
-            self._layers(pb, R, ids_c, pos_c, base_c, cap_c, "batch", st, crec, rows_d, pf)
+            pf = PrefillPlan([(sent[t], lo, n) for t, lo, n in groups], kexp, vexp)
+            self._layers(pb, R, ids_all[s:e], pos_all[s:e], base_all[s:e], cap_all[s:e], "batch", st, crec, rows_d, pf)
             for r in crec or ():
                 for j, t in enumerate(r[2:]):  # scatter the last-token rows to their sequences
                     key = (r[0], r[1], j)
                     if key not in acc:
                         acc[key] = torch.zeros((self.B,) + tuple(t.shape[1:]), dtype=t.dtype, device=dev)
-                    acc[key].index_copy_(0, slot_t.to(dev)[which], t)
-            if rows.numel():
+                    acc[key].index_copy_(0, slot_d[which], t)
+            if n_last:
                 last_h.index_copy_(0, which, pb.h[rows_d])
                 last_xn.index_copy_(0, which, pb.xn[rows_d])
         # final norm is fused into the last layer's combine (pb.xn); lm_head + argmax
@@ -645,11 +703,10 @@ class DecodeEngine:
         call("dsv2_gemm_bf16", ptr(last_xn), c.hidden, 0, k, c.hidden, ptr(self.w.lm_head), 0, c.vocab, 1, None,
              0, ptr(logits), c.vocab, 0, LINEAR_OUT_F32, st)
         call("dsv2_argmax_f32", ptr(logits), k, c.vocab, ptr(ids), None, st)
-        slot_d = slot_t.to(dev)
         if not whole:
             self.logits.index_copy_(0, slot_d, logits)
             self.ids.index_copy_(0, slot_d, ids)
-        self.cache.pos.index_copy_(0, slot_d, torch.tensor(lens, dtype=torch.int32, device=dev))
+        self.cache.pos.index_copy_(0, slot_d, sent[i_lens])
         for b, n in zip(slots, lens):
             self._host_pos[b] = n
         if record is not None:

@@ -392,3 +392,16 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
     assert len(groups) == 1
     t, lo, n = prefill_tiles(seq, posv, bases)
     assert torch.equal(groups[0][0], t) and groups[0][1:] == (lo, n)
+
+
+def test_chunk_segments_equal_the_rows_own_runs():
+    """The chunk plan from prompt lengths alone equals the one read off the chunk's per-row
+    sequence and position tensors, for every cut of ragged prompts."""
+    from dsv2lite.engine import _chunk_segments, _segments
+
+    lens = [5, 1, 17, 9]
+    seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(lens)])
+    posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
+    for s in range(sum(lens)):
+        for e in range(s + 1, sum(lens) + 1):
+            assert _chunk_segments(lens, s, e) == _segments(seq[s:e], posv[s:e])

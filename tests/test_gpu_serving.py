@@ -83,3 +83,21 @@ def test_retired_slot_wraps_inside_its_capacity(weights):
     with pytest.raises(ValueError, match="does not fit"):
         eng.insert(1, _prompts([12], 4)[0])
     assert eng.insert(1, _prompts([4], 4)[0]) >= 0 and eng.free_slots == []
+
+
+@pytest.mark.parametrize("where", ["host", "mixed"])
+def test_prefill_takes_prompts_from_host_or_device_alike(weights, where):
+    """Prompts on the host (sent in one copy with the chunk plan) give bitwise the state of the
+    same prompts on the device, over chunks in which no, one and several prompts end."""
+    import dsv2lite
+
+    prompts = _prompts([40, 3, 5, 17], 3)
+    other = [p.cpu() if where == "host" or i % 2 else p for i, p in enumerate(prompts)]
+    states = []
+    for ps in (prompts, other):
+        eng = dsv2lite.DecodeEngine(weights, [64] * 4, family="batch", max_prefill_rows=16, moe_tile=16)
+        eng.prefill(ps)
+        torch.cuda.synchronize()
+        states.append((eng.logits.clone(), eng.ids.clone(), eng.cache.pos.clone(), eng.cache.data.clone()))
+    for a, b in zip(*states):
+        assert torch.equal(a, b)
