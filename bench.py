@@ -790,7 +790,7 @@ def run_config(key, w, args, cfg, dev, expert_dtype: str = "bf16") -> dict:
     ctx_avg = sum(n + 1 + (steps - 1) / 2 for n in lens)
     sb = step_bytes(cfg, n_exp, ctx_avg, B, expert_dtype == "fp8")
     _log(f"config {key}: timed {steps} graph replays: {ms:.3f} ms/step, {value:.1f} tok/s")
-    roof = time_dominant_kernel(eng, family)
+    roof = time_dominant_kernel(eng, eng.step_family)
     roof["traffic"], roof["traffic_source"] = measured_traffic(key, roof["kernel"])
     prof = STEP_PROFILES.get(key) if expert_dtype == "bf16" else None
     ins = in_step_timing(prof, roof["kernel"]) if prof else None
@@ -798,10 +798,10 @@ def run_config(key, w, args, cfg, dev, expert_dtype: str = "bf16") -> dict:
         ins["frac"] = roof["bytes_per_launch"] / (ins["avg_us"] * 1e-6) / HBM_PEAK
         roof["in_step"] = ins
     pos_now = eng.cache.pos.cpu().tolist()
-    others = time_other_kernels(eng, family, [p + 1 for p in pos_now])
+    others = time_other_kernels(eng, eng.step_family, [p + 1 for p in pos_now])
     res = {"workload": spec["workload"] + (", e4m3 expert weights" if expert_dtype == "fp8" else ""),
            "expert_dtype": expert_dtype, "global_batch": B, "seq_len": max(lens), "kernel_family": family,
-           "mla_path": args.mla_path if family == "small" else "split", "prompt_tokens": sum(lens),
+           "mla_path": args.mla_path if eng.step_family == "small" else "split", "prompt_tokens": sum(lens),
            "tok_s": value, "ms_per_step": ms, "steps": steps, "warmup": warm, "kernels_per_step": eng.kernels_per_step,
            "roofline": roof,
            "other_kernels": others,

@@ -10,7 +10,8 @@ Kernel families (``--kernel-family``, src/run.py:53-65):
   small -- VALU GEMV with fused RMSNorm prologue and residual epilogue; fused
            MLA prepare (RoPE + cache write + W_UK absorption) and fused
            combine + W_UV; route-local MoE over 6 routed + 2 shared "half"
-           experts with a deterministic in-workgroup top-6 combine.
+           experts with a deterministic in-workgroup top-6 combine.  From SMALL_BATCH_ROWS
+           rows its step runs the batch family's kernels.
   batch -- bf16 MFMA grouped GEMM for every projection (heads-batched W_UK /
            W_UV), deterministic expert bucketing, expert-grouped gate_up+SwiGLU
            and down on MFMA, fused combine + shared + residual + next RMSNorm.
@@ -37,6 +38,14 @@ from .weights import ModelWeights
 BF16 = torch.bfloat16
 FAMILIES = ("small", "batch")
 FUSED_MLA_MAX_CTX = 2048
+# small family (default MLA path): from this many rows the step runs the batch family's kernels.
+# The GEMV kernels read a routed expert's weights once per row that chose it and repeat the
+# dense dot products per row on the VALU (lm_head at 8 rows 174 us against 86 on MFMA, dense
+# gate_up 65 against 19, the expert launches 160 against 121).  Measured on MI355X, four-layer
+# steps (contexts 24..600 / 300..1800), small against batch kernels: 4 rows 548 vs 591 us / 613 vs
+# 604, 5 rows 696 vs 615 / 755 vs 599, 8 rows 983 vs 707 / 1104 vs 731, 12 rows 1447 vs 769; e4m3
+# experts 4 rows 452 vs 471 / 518 vs 485, 5 rows 575 vs 494 / 643 vs 475
+SMALL_BATCH_ROWS = 5
 # batch family: up to this many rows the router runs as logits over 16 workgroups per token
 # plus a one-wave top-6 per row (64 rows: 8.3 us vs 11.1 us for one workgroup per token on
 # MI355X); above it one workgroup per token (256 rows: 11.4 us vs 14.7 us)
@@ -308,6 +317,8 @@ class DecodeEngine:
         self.cfg = cfg
         self.w = weights
         self.family = family
+        self.step_family = "batch" if family == "small" and mla_path == "absorb" and \
+            len(capacities) >= SMALL_BATCH_ROWS else family
         self.expert_dtype = expert_dtype
         self.device = torch.device(device)
         self.B = len(capacities)
@@ -317,12 +328,15 @@ class DecodeEngine:
         self.scale = cfg.softmax_scale
         self.ids = torch.zeros(self.B, dtype=torch.int64, device=device)
         self.logits = torch.empty(self.B, cfg.vocab, dtype=torch.float32, device=device)
-        self.buf = RowBuffers(cfg, self.B, family, self.max_pos, device)
+        self.buf = RowBuffers(cfg, self.B, self.step_family, self.max_pos, device)
         if family == "batch" and moe_tile is not None:
             self.buf.set_tile_tokens(self._fit_tile(moe_tile))
             self._moe_tiles_tuned = True
-        elif family == "batch":
+        elif self.step_family == "batch":
             self.buf.set_tile_tokens(self._fit_tile(self.buf.tile_tokens))
+            # a few rows of the small family keep this tile whatever they route to, so a row's
+            # results do not depend on the batch it was captured with
+            self._moe_tiles_tuned = family == "small" and self.B <= 16
         self._amax = torch.empty(max(0, _hip.lib.dsv2_lm_head_argmax_workspace_size(min(self.B, 8))),
                                  dtype=torch.uint8, device=device)
         # small family: one fused workgroup per (row, head) while contexts are short; the
@@ -582,9 +596,9 @@ class DecodeEngine:
         next ids into self.ids, advances cache.pos.  No host synchronisation."""
         self._check_room()
         st = _hip.stream_ptr(self.device)
-        self._layers(self.buf, self.B, self.ids, self.cache.pos, self.cache.base, self.cache.cap, self.family, st,
+        self._layers(self.buf, self.B, self.ids, self.cache.pos, self.cache.base, self.cache.cap, self.step_family, st,
                      record)
-        self._head(self.buf, self.family, st, self.cache.pos)
+        self._head(self.buf, self.step_family, st, self.cache.pos)
         self._host_pos = [p + 1 for p in self._host_pos]
 
     def prefill(self, prompts: list[torch.Tensor], record: list | None = None) -> torch.Tensor:
@@ -731,7 +745,7 @@ class DecodeEngine:
         (state restored afterwards), like the reference's tile selection before capture
         (moe_batch.py:596-657) but without timing runs: the median over MoE layers of
         routing_load, mapped by tile_tokens_for_load.  Returns the tile."""
-        if self.family != "batch":
+        if self.step_family != "batch":
             return 0
         snap = self.snapshot()
         rec: list = []
@@ -750,7 +764,7 @@ class DecodeEngine:
         family first picks its MoE token tile from one eager step (tune_moe_tiles).  Sets
         kernels_per_step to the number of nodes of the captured graph (every node is a kernel
         launch: the step records no copies or memsets)."""
-        if self.family == "batch" and not getattr(self, "_moe_tiles_tuned", False):
+        if self.step_family == "batch" and not getattr(self, "_moe_tiles_tuned", False):
             self.tune_moe_tiles()
         saved = list(self._host_pos)
         g = torch.cuda.CUDAGraph(keep_graph=True)

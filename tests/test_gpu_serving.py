@@ -101,3 +101,30 @@ def test_prefill_takes_prompts_from_host_or_device_alike(weights, where):
         states.append((eng.logits.clone(), eng.ids.clone(), eng.cache.pos.clone(), eng.cache.data.clone()))
     for a, b in zip(*states):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows", [4, 5, 8])
+def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
+    """The small family below and from the row count at which its step runs the batch family's
+    kernels: graph replay equals the eager step bitwise, and a sequence decodes to the same bits
+    whatever prompts share its batch."""
+    import dsv2lite
+
+    mine = _prompts([11], 7)[0]
+    got = []
+    for seed in (8, 9):
+        eng = dsv2lite.DecodeEngine(weights, [32] * rows, family="small")
+        eng.prefill([mine] + _prompts([3 + i for i in range(rows - 1)], seed))
+        snap = eng.snapshot()
+        eng.step()
+        eager = eng.logits.clone()
+        eng.restore(snap)
+        eng.capture()
+        eng.restore(snap)
+        for i in range(3):
+            eng.replay()
+            if i == 0:
+                assert torch.equal(eng.logits, eager)
+        eng.check_errors()
+        got.append(eng.logits[0].clone())
+    assert torch.equal(*got)

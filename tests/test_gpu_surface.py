@@ -421,12 +421,14 @@ def test_expanded_attention_tile_edges(B, H, L, pos, Dq, Dv):
     assert rel_err(c(out), torch.softmax(s, -1) @ vd) < 4e-3
 
 
-@pytest.mark.parametrize("tokens", [853, 854, 1024])
-def test_grouped_moe_wrapper_tile_threshold(tokens):
-    """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds,
-    experts unevenly loaded (one empty), against fp32 torch; three bf16 roundings (SwiGLU, expert
+@pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe", n) for n in (853, 854, 1024)]
+                         + [("batched_grouped_routed_moe_route_gemv", n) for n in (6, 7)])
+def test_grouped_moe_wrapper_tile_threshold(fn, tokens):
+    """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds, the
+    route-local form below and above the tokens it hands on, experts unevenly loaded (one empty), against fp32 torch; three bf16 roundings (SwiGLU, expert
     output, sum) of about 2^-9 each: 1e-2."""
-    from triton_kernels.moe_batch import PackedRoutedExperts, batched_grouped_routed_moe
+    from triton_kernels import moe_small_gemv
+    from triton_kernels.moe_batch import PackedRoutedExperts
 
     I = 128
     gu, dn = rnd(64, 2 * I, 2048, seed=80, std=0.02), rnd(64, 2048, I, seed=81, std=0.05)
@@ -435,7 +437,7 @@ def test_grouped_moe_wrapper_tile_threshold(tokens):
     logits = torch.randn(tokens, 64, generator=g) + torch.linspace(-2, 2, 64)
     logits[:, 5] = -1e9
     w, ids = torch.softmax(logits, -1).topk(6, -1)
-    out = batched_grouped_routed_moe(x, ids.to(DEV), w.to(DEV), PackedRoutedExperts(gu, dn, 2048, I, 64, 6))
+    out = getattr(moe_small_gemv, fn)(x, ids.to(DEV), w.to(DEV), PackedRoutedExperts(gu, dn, 2048, I, 64, 6))
     ref = torch.zeros(tokens, 2048)
     xc = c(x)
     for e in range(64):
