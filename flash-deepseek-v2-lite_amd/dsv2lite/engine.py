@@ -142,6 +142,7 @@ def _group_tiles(segs, bases: list[int], tile: int) -> tuple[list[tuple[int, int
         lo = bases[s] if lo is None else min(lo, bases[s])
         last = bases[s] + p_first + cnt
         hi = last if hi is None else max(hi, last)
+    out.sort(key=lambda t: t[1] + t[2])  # by the keys they attend: the kernel takes the last first
     return out, int(lo), int(hi - lo)
 
 

@@ -1205,3 +1205,41 @@ def test_grouped_large_tile_token_counts(inter):
     for a, b in zip(got[256], got[64]):
         assert rel_err(a.float(), b.float()) < 2 ** -7
         assert (a == b).float().mean() > 0.9
+
+
+@pytest.mark.parametrize("lens", [[1], [64], [65], [128, 129, 31, 32, 33], [700]])
+def test_mla_prefill_query_tile_sizes_agree_bitwise(lens):
+    """Few query tiles run as halves of 64 queries, 32 and more as whole tiles: the same sequences
+    alone and beside enough one-token sequences for whole tiles give the same bits, and both are
+    within 1e-2 of fp32 attention (bf16 probabilities and output, 2^-9 each)."""
+    from dsv2lite.engine import prefill_tiles
+
+    outs = []
+    for extra in (0, 33):
+        ls = lens + [1] * extra
+        bases = [0]
+        for n in ls[:-1]:
+            bases.append(bases[-1] + n)
+        R, total = sum(ls), sum(ls)
+        seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(ls)])
+        posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in ls])
+        tiles, lo, nexp = prefill_tiles(seq, posv, bases)
+        assert (tiles.shape[0] >= 32) == (extra > 0)
+        full = total if extra else total + 33  # the same leading rows in both
+        cache, ke, ve = rnd(full, 576, seed=210), rnd(full, 16, 128, seed=211), rnd(full, 16, 128, seed=212)
+        qkva, qrope = rnd(full, 3648, seed=213), rnd(full, 16, 576, seed=214)
+        out = torch.full((full, 2048), float("nan"), dtype=BF, device=DEV)
+        td = tiles.to(DEV)
+        call("dsv2_mla_prefill_attention", qkva.data_ptr(), 3648, qrope.data_ptr(), 16 * 576, R, cache.data_ptr(), full,
+             ke.data_ptr(), ve.data_ptr(), lo, nexp, td.data_ptr(), td.shape[0], 0.1147, out.data_ptr(), 2048, st())
+        outs.append(out[:sum(lens)].clone())
+    assert torch.equal(*outs)
+    at = 0
+    for n in lens:
+        q = torch.cat([qkva[at:at + n, :3072].view(n, 16, 192)[..., :128], qrope[at:at + n, :, 512:]], -1).float()
+        k = torch.cat([ke[at:at + n], cache[at:at + n, None, 512:].expand(-1, 16, -1)], -1).float()
+        s = torch.einsum("qhd,khd->hqk", q, k) * 0.1147
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -math.inf)
+        ref = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), ve[at:at + n].float())
+        assert rel_err(outs[0][at:at + n].float().view(n, 16, 128), ref) < 1e-2
+        at += n
