@@ -59,18 +59,20 @@ def plan_splits(rows: int, max_ctx: int, target_wgs: int = 256) -> tuple[int, in
     most ONE_SPLIT_MAX_CTX tokens (measured on MI355X, whole decode steps, against the
     multi-split plan below: bsz=64 x 57-token caches 2.809 -> 2.726 ms, bsz=64 x 233 6.958 ->
     6.901, bsz=128 x 233 7.941 -> 7.832; at 433 tokens one split loses, 7.013 -> 7.101);
-    else about target_wgs workgroups,
-    split_tokens a multiple of 32, at most 64 splits per row.  256 = one workgroup per CU;
-    each streams its split with two tiles in flight.  Measured on MI355X over the whole
-    decode step against 512: bsz=256 x 2048-token prompts 22.72k vs 22.44k tok/s, bsz=64 x
-    U[256,1024] 8.80k vs 8.70k, reference workload 52.6k vs 51.3k (bsz=256) and 22.0k vs
-    22.0k (bsz=64); 128 (8.55k at bsz=64) and 1024 (bsz=256 x 2098 tokens: 118 vs 109 us per
-    layer) are slower.  Rows of very unequal lengths want more, shorter splits (bsz=128 x
-    U[256,8192]: 512 -> 2048-token splits 132 us, 256 -> 4064-token splits 171 us); capping
-    the split at 2048 tokens instead cost the equal-length bsz=256 step 8%."""
+    else the most splits per row (at most 64, split_tokens a multiple of 32) that leave at most
+    target_wgs workgroups: 256 = one per CU, each streaming its split with two tiles in flight.
+    A few more than 256 make some CUs run two while the rest run one: attention calls of 96 rows
+    x 3,301 tokens 119.8 us with 288, 106.5 with 192, 107.8 with 384; 40 x 6,001 97.5 with 280,
+    90.9 with 200; 70 x 1,601 72.6 with 280, 64.3 with 210.  Where that leaves one split per row
+    and under 171 rows, three (two workgroups on most CUs): 140 rows x 1,601 tokens 108 -> 95 us,
+    160 108 -> 101, but 180 109 -> 119.  Rows of very unequal lengths want more, shorter splits
+    (bsz=128 x U[256,8192]: 512 -> 2048-token splits 132 us, 256 -> 4064-token splits 171 us);
+    capping the split at 2048 tokens instead cost the equal-length bsz=256 step 8%."""
     if max_ctx <= ONE_SPLIT_MAX_CTX:
         return max(32, math.ceil(max_ctx / 32) * 32), 1
-    per_row = max(1, min(64, math.ceil(target_wgs / max(rows, 1))))
+    per_row = max(1, min(64, target_wgs // max(rows, 1)))
+    if per_row == 1 and target_wgs // 2 < rows and 3 * rows <= 2 * target_wgs:
+        per_row = 3
     split = max(32, math.ceil(math.ceil(max_ctx / per_row) / 32) * 32)
     split = max(split, math.ceil(max_ctx / 64 / 32) * 32)
     return split, math.ceil(max_ctx / split)

@@ -1243,3 +1243,26 @@ def test_mla_prefill_query_tile_sizes_agree_bitwise(lens):
         ref = torch.einsum("hqk,khd->qhd", torch.softmax(s, -1), ve[at:at + n].float())
         assert rel_err(outs[0][at:at + n].float().view(n, 16, 128), ref) < 1e-2
         at += n
+
+
+@pytest.mark.parametrize("split,lens", [(32, [1, 32, 33, 64, 65, 97]), (96, [95, 96, 97, 193, 289, 300]),
+                                        (160, [161, 320, 321, 479, 480, 500])])
+def test_mla_decode_equal_pieces(split, lens):
+    """Rows at and around multiples of split_tokens (cut into equal pieces of whole tiles, none empty)
+    against the one-split decode of the same rows: the probabilities are bf16 in both, rounded
+    against another running maximum, and the result is one bf16 round (2^-8 each)."""
+    B, cap = len(lens), 512
+    q, cache = rnd(B, 16, 576, seed=220), rnd(B * cap, 576, seed=221)
+    base = torch.arange(B, device=DEV) * cap
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    capd = torch.full((B,), cap, dtype=torch.int32, device=DEV)
+    ns = max(-(-n // split) for n in lens)
+    part_o = torch.full((B, ns, 16, 512), float("nan"), device=DEV)
+    part_ml = torch.full((B, ns, 16, 2), float("nan"), device=DEV)
+    outs = [torch.empty(B, 16, 512, dtype=BF, device=DEV) for _ in range(2)]
+    P = lambda t: t.data_ptr()  # noqa: E731
+    call("dsv2_mla_decode", P(q), P(cache), P(base), P(pos), P(capd), B, split, ns, 0.1147, P(part_o), P(part_ml), st())
+    call("dsv2_mla_combine", P(part_o), P(part_ml), P(pos), P(capd), B, split, ns, None, P(outs[0]), 8192, st())
+    call("dsv2_mla_decode_rows", P(q), P(cache), P(base), P(pos), P(capd), B, 0.1147, P(outs[1]), 8192, st())
+    assert torch.isfinite(outs[0].float()).all()
+    assert rel_err(outs[0].float(), outs[1].float()) < 2 ** -7
