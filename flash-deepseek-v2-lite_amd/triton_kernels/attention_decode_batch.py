@@ -184,14 +184,17 @@ def _attention_decode(family: str, hidden_states, cos, sin, position_ids, cache_
         call("dsv2_gemv_bf16", P(attn2), HID, B, HID, P(packed.w_o), HID, None, 0.0, None, 0, P(out2), HID, 0, st)
         return ws.out
     call("dsv2_gemm_bf16", P(x), HID, 0, B, HID, P(packed.w_qkva), 0, QKVA, 1, None, 0, P(ws.qkva), QKVA, 0, 0, st)
-    call("dsv2_mla_prepare", P(ws.qkva), QKVA, B, P(ws.pos), P(ws.base), P(ws.cap), P(packed.kv_norm_weight),
-         packed.kv_norm_eps, P(cos2), P(sin2), max_pos, None, P(key_cache), P(ws.q), P(ws.status), st)
-    call("dsv2_gemm_bf16", P(ws.qkva), QKVA, NOPE + ROPE, B, NOPE, P(packed.w_ukt), LAT * NOPE, LAT, NH, None, 0,
-         P(ws.q), NH * ROW, ROW, 0, st)
-    call("dsv2_mla_decode", P(ws.q), P(key_cache), P(ws.base), P(ws.pos), P(ws.cap), B, ws.split, ws.nsplit,
-         float(softmax_scale), P(ws.part_o), P(ws.part_ml), st)
-    call("dsv2_mla_combine", P(ws.part_o), P(ws.part_ml), P(ws.pos), P(ws.cap), B, ws.split, ws.nsplit, None,
-         P(ws.olat), NH * LAT, st)
+    # the new cache row, RoPE and the W_UK absorption in one launch; one split per row needs no merge
+    call("dsv2_mla_prepare_qlat", P(ws.qkva), QKVA, B, P(ws.pos), P(ws.base), P(ws.cap), P(packed.kv_norm_weight),
+         packed.kv_norm_eps, P(cos2), P(sin2), max_pos, P(packed.w_ukt), P(key_cache), P(ws.q), P(ws.status), st)
+    if ws.nsplit == 1:
+        call("dsv2_mla_decode_rows", P(ws.q), P(key_cache), P(ws.base), P(ws.pos), P(ws.cap), B, float(softmax_scale),
+             P(ws.olat), NH * LAT, st)
+    else:
+        call("dsv2_mla_decode", P(ws.q), P(key_cache), P(ws.base), P(ws.pos), P(ws.cap), B, ws.split, ws.nsplit,
+             float(softmax_scale), P(ws.part_o), P(ws.part_ml), st)
+        call("dsv2_mla_combine", P(ws.part_o), P(ws.part_ml), P(ws.pos), P(ws.cap), B, ws.split, ws.nsplit, None,
+             P(ws.olat), NH * LAT, st)
     call("dsv2_gemm_bf16", P(ws.olat), NH * LAT, LAT, B, LAT, P(packed.w_uv), VD * LAT, VD, NH, None, 0, P(attn2),
          HID, VD, 0, st)
     call("dsv2_gemm_bf16", P(attn2), HID, 0, B, HID, P(packed.w_o), 0, HID, 1, None, 0, P(out2), HID, 0, 0, st)
