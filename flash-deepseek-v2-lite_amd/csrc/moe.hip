@@ -186,6 +186,7 @@ struct RouteGateupArgs {
   int gu_blocks, nr, hbuf_routes, inter;
   const bf16_t* xn;
   int32_t* ids;          // [rows, 6]: read (logits == null) or written (logits != null)
+  int id_step;           // int32 words per id read: 1, or 2 for the low words of int64 ids
   const float* logits;   // non-null: the row's fp32 router logits, ranked here
   float scaling;
   float* wts;            // written with ids when logits != null
@@ -245,7 +246,7 @@ __device__ __forceinline__ int route_expert(const RouteGateupArgs& a, int b, int
       }
     }
   } else if (s < kTopK) {
-    e = min(max(a.ids[b * kTopK + s], 0), kE - 1);
+    e = min(max(a.ids[(b * kTopK + s) * a.id_step], 0), kE - 1);
   }
   return e;
 }
@@ -414,8 +415,8 @@ static int launch_route_gateup(RouteGateupArgs& a, int rows, hipStream_t st, con
   return dsv2_launch_status(what);
 }
 
-extern "C" int dsv2_moe_route_gateup(const void* xn, int rows, const int32_t* ids, const void* w_gate_up,
-                                     const void* sh_gate_up, int inter, void* hbuf, void* stream) {
+static int route_gateup_ids(const void* xn, int rows, const int32_t* ids, int id_step, const void* w_gate_up,
+                            const void* sh_gate_up, int inter, void* hbuf, void* stream) {
   DSV2_REQUIRE(xn && ids && w_gate_up && hbuf, DSV2_E_NULL, "moe_route_gateup: null pointer");
   const int nr = sh_gate_up ? kTopK + 2 : kTopK;
   DSV2_REQUIRE(rows >= 0 && (int64_t)rows * nr <= 65535 && inter > 0 && inter % 8 == 0, DSV2_E_SHAPE,
@@ -429,10 +430,22 @@ extern "C" int dsv2_moe_route_gateup(const void* xn, int rows, const int32_t* id
   a.inter = inter;
   a.xn = (const bf16_t*)xn;
   a.ids = const_cast<int32_t*>(ids);
+  a.id_step = id_step;
   a.wgu = (const bf16_t*)w_gate_up;
   a.shgu = (const bf16_t*)sh_gate_up;
   a.hbuf = (bf16_t*)hbuf;
   return launch_route_gateup(a, rows, (hipStream_t)stream, "moe_route_gateup");
+}
+
+extern "C" int dsv2_moe_route_gateup(const void* xn, int rows, const int32_t* ids, const void* w_gate_up,
+                                     const void* sh_gate_up, int inter, void* hbuf, void* stream) {
+  return route_gateup_ids(xn, rows, ids, 1, w_gate_up, sh_gate_up, inter, hbuf, stream);
+}
+
+extern "C" int dsv2_moe_route_gateup_i64(const void* xn, int rows, const int64_t* ids, const void* w_gate_up,
+                                         const void* sh_gate_up, int inter, void* hbuf, void* stream) {
+  return route_gateup_ids(xn, rows, reinterpret_cast<const int32_t*>(ids), 2, w_gate_up, sh_gate_up, inter, hbuf,
+                          stream);
 }
 
 extern "C" int dsv2_moe_route_gateup_logits(const void* xn, int rows, const float* logits, float scaling,
@@ -502,7 +515,7 @@ extern "C" int dsv2_moe_route_gateup_logits_fp8(const void* xn, int rows, const 
 // ---------------------------------------------------------------------------
 template <int NR>
 __global__ __launch_bounds__(256) void route_down_kernel(const bf16_t* __restrict__ hbuf,
-                                                         const int32_t* __restrict__ ids,
+                                                         const int32_t* __restrict__ ids, int id_step,
                                                          const float* __restrict__ wts,
                                                          const bf16_t* __restrict__ wd,
                                                          const bf16_t* __restrict__ shd, int inter, int hbuf_routes,
@@ -521,7 +534,7 @@ __global__ __launch_bounds__(256) void route_down_kernel(const bf16_t* __restric
   // where used).
   int eid[2];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) eid[q] = ids[b * kTopK + min(2 * wv + q, kTopK - 1)];
+  for (int q = 0; q < 2; ++q) eid[q] = ids[(b * kTopK + min(2 * wv + q, kTopK - 1)) * id_step];
   const int jr = j0 + (threadIdx.x & 1);
   bf16_t resb = 0, shb = 0;
   resb = (res ? res : hbuf)[res ? (int64_t)b * kH + jr : 0];
@@ -722,9 +735,9 @@ extern "C" int dsv2_moe_route_down_fp8(const void* hbuf, int rows, const int32_t
   return dsv2_launch_status("moe_route_down_fp8");
 }
 
-extern "C" int dsv2_moe_route_down(const void* hbuf, int rows, const int32_t* ids, const float* weights,
-                                   const void* w_down, const void* sh_down, int inter, int hbuf_routes,
-                                   const void* shared_y, const void* residual, void* out, void* stream) {
+static int route_down_ids(const void* hbuf, int rows, const int32_t* ids, int id_step, const float* weights,
+                          const void* w_down, const void* sh_down, int inter, int hbuf_routes, const void* shared_y,
+                          const void* residual, void* out, void* stream) {
   DSV2_REQUIRE(hbuf && ids && weights && w_down && out, DSV2_E_NULL, "moe_route_down: null pointer");
   DSV2_REQUIRE(rows >= 0 && rows <= 65535 && inter > 0 && inter % 8 == 0 && inter <= 3 * 64 * 8, DSV2_E_SHAPE,
                "moe_route_down: bad shape (inter %% 8 == 0, inter <= 1536)");
@@ -737,13 +750,27 @@ extern "C" int dsv2_moe_route_down(const void* hbuf, int rows, const int32_t* id
   const dim3 grid(kH / 2, rows);
   if (sh_down)
     hipLaunchKernelGGL((route_down_kernel<kTopK + 2>), grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)hbuf,
-                       ids, weights, (const bf16_t*)w_down, (const bf16_t*)sh_down, inter, hbuf_routes, nullptr,
+                       ids, id_step, weights, (const bf16_t*)w_down, (const bf16_t*)sh_down, inter, hbuf_routes, nullptr,
                        (const bf16_t*)residual, (bf16_t*)out);
   else
     hipLaunchKernelGGL((route_down_kernel<kTopK>), grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)hbuf, ids,
-                       weights, (const bf16_t*)w_down, nullptr, inter, hbuf_routes, (const bf16_t*)shared_y,
+                       id_step, weights, (const bf16_t*)w_down, nullptr, inter, hbuf_routes, (const bf16_t*)shared_y,
                        (const bf16_t*)residual, (bf16_t*)out);
   return dsv2_launch_status("moe_route_down");
+}
+
+extern "C" int dsv2_moe_route_down(const void* hbuf, int rows, const int32_t* ids, const float* weights,
+                                   const void* w_down, const void* sh_down, int inter, int hbuf_routes,
+                                   const void* shared_y, const void* residual, void* out, void* stream) {
+  return route_down_ids(hbuf, rows, ids, 1, weights, w_down, sh_down, inter, hbuf_routes, shared_y, residual, out,
+                        stream);
+}
+
+extern "C" int dsv2_moe_route_down_i64(const void* hbuf, int rows, const int64_t* ids, const float* weights,
+                                       const void* w_down, const void* sh_down, int inter, int hbuf_routes,
+                                       const void* shared_y, const void* residual, void* out, void* stream) {
+  return route_down_ids(hbuf, rows, reinterpret_cast<const int32_t*>(ids), 2, weights, w_down, sh_down, inter,
+                        hbuf_routes, shared_y, residual, out, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -771,13 +798,14 @@ __device__ __forceinline__ int chunk_rank(int e, int lane, bool& last) {
   last = __popcll(same & ~below) == 1;
   return __popcll(same & below);
 }
-__device__ __forceinline__ int route_rank(const int32_t* __restrict__ ids, int r, int R, int lane, int& e,
-                                          bool& last) {
-  e = r < R ? min(max(ids[r], 0), kE - 1) : kE;
+__device__ __forceinline__ int route_rank(const int32_t* __restrict__ ids, int id_step, int r, int R, int lane,
+                                          int& e, bool& last) {
+  e = r < R ? min(max(ids[r * id_step], 0), kE - 1) : kE;
   return chunk_rank(e, lane, last);
 }
 
-__global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict__ ids, int R, int tile_tokens,
+__global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict__ ids, int id_step, int R,
+                                                      int tile_tokens,
                                                       int32_t* __restrict__ sorted_routes,
                                                       int32_t* __restrict__ route_pos, int32_t* __restrict__ tiles,
                                                       int32_t* __restrict__ num_tiles) {
@@ -791,7 +819,7 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict_
   const int32_t* idp = R > 0 ? ids : num_tiles;
   int ek[2], bk[2] = {0, 0};
 #pragma unroll
-  for (int k = 0; k < 2; ++k) ek[k] = idp[max(min((wv + 16 * k) * 64 + lane, R - 1), 0)];
+  for (int k = 0; k < 2; ++k) ek[k] = idp[max(min((wv + 16 * k) * 64 + lane, R - 1), 0) * id_step];
   for (int i = tid; i < nchunks * kE; i += 1024) hist[i / kE][i % kE] = 0;
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -810,7 +838,7 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict_
       e = ek[1];
       before = bk[1] = chunk_rank(e, lane, last);
     } else {
-      before = route_rank(ids, c * 64 + lane, R, lane, e, last);
+      before = route_rank(ids, id_step, c * 64 + lane, R, lane, e, last);
     }
     if (c * 64 + lane < R && last) hist[c][e] = (uint16_t)(before + 1);
   }
@@ -853,7 +881,7 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict_
       before = bk[1];
     } else {
       bool last;
-      before = route_rank(ids, r, R, lane, e, last);
+      before = route_rank(ids, id_step, r, R, lane, e, last);
     }
     if (r < R) {
       const int p = start[e] + hist[c][e] + before;
@@ -875,15 +903,26 @@ __global__ __launch_bounds__(1024) void bucket_kernel(const int32_t* __restrict_
   }
 }
 
-extern "C" int dsv2_moe_bucket(const int32_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
-                               int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* stream) {
+static int bucket_ids(const int32_t* ids, int id_step, int rows, int tile_tokens, int32_t* sorted_routes,
+                      int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* stream) {
   DSV2_REQUIRE(ids && sorted_routes && route_pos && tiles && num_tiles, DSV2_E_NULL, "moe_bucket: null pointer");
   DSV2_REQUIRE(rows >= 0 && rows * kTopK <= kMaxRoutes && tile_tokens >= 1 && tile_tokens <= 256, DSV2_E_SHAPE,
                "moe_bucket: rows*6 must be <= %d (got %d)", kMaxRoutes, rows * kTopK);
   DSV2_REQUIRE(dsv2_aligned16(tiles), DSV2_E_ALIGN, "moe_bucket: tiles must be 16-byte aligned");
-  hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, rows * kTopK, tile_tokens,
-                     sorted_routes, route_pos, tiles, num_tiles);
+  hipLaunchKernelGGL(bucket_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, id_step, rows * kTopK,
+                     tile_tokens, sorted_routes, route_pos, tiles, num_tiles);
   return dsv2_launch_status("moe_bucket");
+}
+
+extern "C" int dsv2_moe_bucket(const int32_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
+                               int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* stream) {
+  return bucket_ids(ids, 1, rows, tile_tokens, sorted_routes, route_pos, tiles, num_tiles, stream);
+}
+
+extern "C" int dsv2_moe_bucket_i64(const int64_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
+                                   int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* stream) {
+  return bucket_ids(reinterpret_cast<const int32_t*>(ids), 2, rows, tile_tokens, sorted_routes, route_pos, tiles,
+                    num_tiles, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -893,7 +932,7 @@ extern "C" int dsv2_moe_bucket(const int32_t* ids, int rows, int tile_tokens, in
 // scatter (one wave per chunk).  The histograms live in the caller's workspace (int32
 // [chunks][64], then the 64 expert starts).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void bucket_hist_kernel(const int32_t* __restrict__ ids, int R,
+__global__ __launch_bounds__(1024) void bucket_hist_kernel(const int32_t* __restrict__ ids, int id_step, int R,
                                                            int32_t* __restrict__ hist) {
   __shared__ int cnt[16][kE];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -901,7 +940,7 @@ __global__ __launch_bounds__(1024) void bucket_hist_kernel(const int32_t* __rest
   const bool live = c < nchunks;  // per wave
   int e = kE, before = 0;
   bool last = false;
-  if (live) before = route_rank(ids, c * 64 + lane, R, lane, e, last);
+  if (live) before = route_rank(ids, id_step, c * 64 + lane, R, lane, e, last);
   cnt[wv][lane] = 0;
   __syncthreads();  // the lanes' count writes below land after every zero
   if (live && c * 64 + lane < R && last) cnt[wv][e] = before + 1;
@@ -980,7 +1019,7 @@ __global__ __launch_bounds__(1024) void bucket_scan_kernel(int R, int tile_token
   }
 }
 
-__global__ __launch_bounds__(1024) void bucket_scatter_kernel(const int32_t* __restrict__ ids, int R,
+__global__ __launch_bounds__(1024) void bucket_scatter_kernel(const int32_t* __restrict__ ids, int id_step, int R,
                                                               const int32_t* __restrict__ hist,
                                                               int32_t* __restrict__ sorted_routes,
                                                               int32_t* __restrict__ route_pos) {
@@ -990,7 +1029,7 @@ __global__ __launch_bounds__(1024) void bucket_scatter_kernel(const int32_t* __r
   const int r = c * 64 + lane;
   int e;
   bool last;
-  const int before = route_rank(ids, r, R, lane, e, last);
+  const int before = route_rank(ids, id_step, r, R, lane, e, last);
   if (r < R) {
     const int p = hist[(int64_t)nchunks * kE + e] + hist[(int64_t)c * kE + e] + before;
     sorted_routes[p] = r;
@@ -1003,9 +1042,9 @@ extern "C" int64_t dsv2_moe_bucket_workspace_size(int rows) {
   return (nchunks + 1) * kE * (int64_t)sizeof(int32_t);
 }
 
-extern "C" int dsv2_moe_bucket_wide(const int32_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
-                                    int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* workspace,
-                                    int64_t workspace_bytes, void* stream) {
+static int bucket_wide_ids(const int32_t* ids, int id_step, int rows, int tile_tokens, int32_t* sorted_routes,
+                           int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* workspace,
+                           int64_t workspace_bytes, void* stream) {
   DSV2_REQUIRE(ids && sorted_routes && route_pos && tiles && num_tiles && workspace, DSV2_E_NULL,
                "moe_bucket_wide: null pointer");
   DSV2_REQUIRE(rows >= 0 && rows * kTopK <= kMaxRoutes && tile_tokens >= 1 && tile_tokens <= 256, DSV2_E_SHAPE,
@@ -1018,11 +1057,26 @@ extern "C" int dsv2_moe_bucket_wide(const int32_t* ids, int rows, int tile_token
   int32_t* hist = reinterpret_cast<int32_t*>(workspace);
   const int groups = (nchunks + 15) / 16;
   hipStream_t st = (hipStream_t)stream;
-  if (groups > 0) hipLaunchKernelGGL(bucket_hist_kernel, dim3(groups), dim3(1024), 0, st, ids, R, hist);
+  if (groups > 0) hipLaunchKernelGGL(bucket_hist_kernel, dim3(groups), dim3(1024), 0, st, ids, id_step, R, hist);
   hipLaunchKernelGGL(bucket_scan_kernel, dim3(1), dim3(1024), 0, st, R, tile_tokens, hist, tiles, num_tiles);
   if (groups > 0)
-    hipLaunchKernelGGL(bucket_scatter_kernel, dim3(groups), dim3(1024), 0, st, ids, R, hist, sorted_routes, route_pos);
+    hipLaunchKernelGGL(bucket_scatter_kernel, dim3(groups), dim3(1024), 0, st, ids, id_step, R, hist,
+                       sorted_routes, route_pos);
   return dsv2_launch_status("moe_bucket_wide");
+}
+
+extern "C" int dsv2_moe_bucket_wide(const int32_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
+                                    int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+  return bucket_wide_ids(ids, 1, rows, tile_tokens, sorted_routes, route_pos, tiles, num_tiles, workspace,
+                         workspace_bytes, stream);
+}
+
+extern "C" int dsv2_moe_bucket_wide_i64(const int64_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
+                                        int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  return bucket_wide_ids(reinterpret_cast<const int32_t*>(ids), 2, rows, tile_tokens, sorted_routes, route_pos, tiles,
+                         num_tiles, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -7,7 +7,7 @@ from __future__ import annotations
 import torch
 
 from . import _hip
-from .moe_batch import (PackedRoutedExperts, _check, batched_grouped_routed_moe, pack_routed_experts,  # noqa: F401
+from .moe_batch import (PackedRoutedExperts, _check, _ids, batched_grouped_routed_moe, pack_routed_experts,  # noqa: F401
                         packed_routed_moe_eager)
 
 # more tokens take the expert-grouped kernels, which read an expert's weights once for all its
@@ -27,15 +27,15 @@ def batched_grouped_routed_moe_route_gemv(x: torch.Tensor, topk_ids: torch.Tenso
     if ROUTE_GEMV_MAX_TOKENS < x.shape[0] <= 8192 and packed.intermediate_size <= 1536:
         return batched_grouped_routed_moe(x, topk_ids, topk_weight, packed)
     x = x.contiguous()
-    ids = topk_ids.to(torch.int32).contiguous()
+    ids, i64 = _ids(topk_ids)
     w = topk_weight.to(torch.float32).contiguous()
     B, I = x.shape[0], packed.intermediate_size
     hbuf = torch.empty(B, 6, I, dtype=torch.bfloat16, device=x.device)
     out = torch.empty(B, 2048, dtype=torch.bfloat16, device=x.device)
     st = _hip.stream_ptr(x.device)
-    _hip.call("dsv2_moe_route_gateup", x.data_ptr(), B, ids.data_ptr(), packed.gate_up_weights.data_ptr(), None, I,
+    _hip.call("dsv2_moe_route_gateup" + i64, x.data_ptr(), B, ids.data_ptr(), packed.gate_up_weights.data_ptr(), None, I,
               hbuf.data_ptr(), st)
-    _hip.call("dsv2_moe_route_down", hbuf.data_ptr(), B, ids.data_ptr(), w.data_ptr(), packed.down_weights.data_ptr(),
+    _hip.call("dsv2_moe_route_down" + i64, hbuf.data_ptr(), B, ids.data_ptr(), w.data_ptr(), packed.down_weights.data_ptr(),
               None, I, 6, None, None, out.data_ptr(), st)
     return out
 

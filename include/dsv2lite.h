@@ -400,6 +400,19 @@ int64_t dsv2_moe_bucket_workspace_size(int rows);
 int dsv2_moe_bucket_wide(const int32_t* ids, int rows, int tile_tokens, int32_t* sorted_routes, int32_t* route_pos,
                          int32_t* tiles, int32_t* num_tiles, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The four entry points that read router ids, for int64 ids (what router_softmax_topk6_triton and
+ * torch.topk return): same arguments and results otherwise. */
+int dsv2_moe_route_gateup_i64(const void* xn, int rows, const int64_t* ids, const void* w_gate_up,
+                              const void* sh_gate_up, int inter, void* hbuf, void* stream);
+int dsv2_moe_route_down_i64(const void* hbuf, int rows, const int64_t* ids, const float* weights, const void* w_down,
+                            const void* sh_down, int inter, int hbuf_routes, const void* shared_y,
+                            const void* residual, void* out, void* stream);
+int dsv2_moe_bucket_i64(const int64_t* ids, int rows, int tile_tokens, int32_t* sorted_routes, int32_t* route_pos,
+                        int32_t* tiles, int32_t* num_tiles, void* stream);
+int dsv2_moe_bucket_wide_i64(const int64_t* ids, int rows, int tile_tokens, int32_t* sorted_routes,
+                             int32_t* route_pos, int32_t* tiles, int32_t* num_tiles, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+
 /* Expert-grouped gate_up + SwiGLU on bf16 MFMA over the tiles of dsv2_moe_bucket:
  *   hsorted[p, :inter] for p in tile = SwiGLU(xn[sorted_routes[p]/6] . W_e^T).
  * tile_tokens 16, 32, 64 or 256 (256: inter % 128 == 0).

@@ -448,6 +448,25 @@ def test_grouped_moe_wrapper_tile_threshold(fn, tokens):
     assert rel_err(c(out), ref) < 1e-2
 
 
+@pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe_route_gemv", 3), ("batched_grouped_routed_moe", 1),
+                                       ("batched_grouped_routed_moe", 400), ("batched_grouped_routed_moe", 1100)])
+def test_routed_moe_takes_int64_and_int32_ids_alike(fn, tokens):
+    """int64 ids are read in place, others cast to int32: the same bits, out-of-range and negative
+    ids (clamped) included."""
+    from triton_kernels import moe_small_gemv
+    from triton_kernels.moe_batch import PackedRoutedExperts
+
+    packed = PackedRoutedExperts(rnd(64, 256, 2048, seed=84, std=0.02), rnd(64, 2048, 128, seed=85, std=0.05), 2048, 128,
+                                 64, 6)
+    x = rnd(tokens, 2048, seed=86)
+    g = torch.Generator().manual_seed(87)
+    ids = torch.stack([torch.randperm(64, generator=g)[:6] for _ in range(tokens)])
+    ids[0, 0], ids[-1, 5] = -3, 70
+    w = torch.rand(tokens, 6, generator=g).to(DEV)
+    a, b = (getattr(moe_small_gemv, fn)(x, ids.to(dt).to(DEV), w, packed) for dt in (torch.int64, torch.int32))
+    assert torch.equal(a, b)
+
+
 # --------------------------------------------------------------------------- capacity guard (C ABI)
 def test_mla_kernels_never_touch_another_rows_slots():
     """Row 0 at pos == cap (full), row 1 with room.  The split-KV path (prepare + decode +
