@@ -38,6 +38,12 @@ from .weights import ModelWeights
 BF16 = torch.bfloat16
 FAMILIES = ("small", "batch")
 FUSED_MLA_MAX_CTX = 2048
+# small family, "absorb": caches up to this many tokens.  Its attention launch gives each of a
+# head's four workgroups every cached token; the split-KV decode spreads them over 64 splits and
+# costs two launches more.  Measured on MI355X, four-layer steps, absorb against split at 128 / 400
+# / 600 / 1100 / 1950 cached tokens: 1 row 260 vs 295 us, 288 vs 286, 299 vs 291, 325 vs 299, 370 vs
+# 314; 4 rows 511 vs 532, 535 vs 524, 550 vs 529, 576 vs 542, 627 vs 559
+ABSORB_MAX_CTX = 640
 # small family (default MLA path): from this many rows the step runs the batch family's kernels.
 # The GEMV kernels read a routed expert's weights once per row that chose it and repeat the
 # dense dot products per row on the VALU (lm_head at 8 rows 174 us against 86 on MFMA, dense
@@ -348,9 +354,10 @@ class DecodeEngine:
         self.spread_mla = family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX and mla_path == "spread"
         # small family, "absorb": the q|kv_a projection also forms the absorbed query in partial
         # sums (dsv2_qkva_absorb_bf16), then one attention launch (dsv2_mla_attend_parts)
-        self.absorb_mla = family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX and mla_path == "absorb"
-        self.mla_path = ("fused" if self.fused_mla else "spread" if self.spread_mla else
-                         "absorb" if self.absorb_mla else "split")
+        self.absorb_mla = self.step_family == "small" and self.max_pos <= ABSORB_MAX_CTX and mla_path == "absorb"
+        # the path asked for, where the cache is short enough for the one- and two-launch paths at
+        # all; "absorb" leaves caches past ABSORB_MAX_CTX to the split-KV decode as well
+        self.mla_path = mla_path if family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX else "split"
         self.max_prefill_rows = max_prefill_rows
         self.graph = None
         self.kernels_per_step = 0  # set by capture()

@@ -79,8 +79,8 @@ def plan_splits(rows: int, max_ctx: int, target_wgs: int = 256) -> tuple[int, in
 
 
 # the small family runs the absorb path (dsv2_qkva_absorb_bf16 + dsv2_mla_attend_parts) while
-# the cache is this short, like the engine (dsv2lite.engine.FUSED_MLA_MAX_CTX); longer caches
-# take the split-KV decode
+# the cache is this short; longer caches take the split-KV decode (from 640 tokens its kernels are
+# the faster ones, but these calls launch eagerly and two launches more cost the host 11 us)
 FUSED_MAX_CTX = 2048
 
 

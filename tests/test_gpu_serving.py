@@ -128,3 +128,23 @@ def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
         eng.check_errors()
         got.append(eng.logits[0].clone())
     assert torch.equal(*got)
+
+
+def test_small_family_absorb_and_split_decode_agree_at_the_threshold(weights):
+    """The small family's attention just below and above the capacity at which "absorb" hands over
+    to the split-KV decode: same prompt, logits within the 2e-2 parity bar of each other."""
+    import dsv2lite
+    from dsv2lite.engine import ABSORB_MAX_CTX
+
+    prompt = _prompts([ABSORB_MAX_CTX - 30], 11)
+    got = []
+    for cap in (ABSORB_MAX_CTX, ABSORB_MAX_CTX + 1):
+        eng = dsv2lite.DecodeEngine(weights, [cap], family="small")
+        assert eng.absorb_mla == (cap == ABSORB_MAX_CTX)
+        eng.prefill(prompt)
+        for _ in range(3):
+            eng.ids.fill_(77)  # the same tokens whatever the logits say
+            eng.step()
+        eng.check_errors()
+        got.append(eng.logits.float().clone())
+    assert float((got[0] - got[1]).abs().max() / got[0].abs().max()) < 2e-2
