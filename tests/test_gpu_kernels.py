@@ -1266,3 +1266,18 @@ def test_mla_decode_equal_pieces(split, lens):
     call("dsv2_mla_decode_rows", P(q), P(cache), P(base), P(pos), P(capd), B, 0.1147, P(outs[1]), 8192, st())
     assert torch.isfinite(outs[0].float()).all()
     assert rel_err(outs[0].float(), outs[1].float()) < 2 ** -7
+
+
+@pytest.mark.parametrize("rows", [1, 1024, 1025, 4099])
+def test_topk6_from_logits_rows_per_workgroup(rows):
+    """One and four rows per workgroup, a partial last workgroup: ids exact (ties to the lower
+    index), weights of the fp32 softmax to 1e-6."""
+    lg = rnd(rows, 64, seed=230, dtype=torch.float32)
+    lg[-1] = lg[-1, 0]  # all tied: experts 0..5
+    ids = torch.full((rows, 6), -1, dtype=torch.int64, device=DEV)
+    w = torch.zeros(rows, 6, device=DEV)
+    call("dsv2_router_topk6_from_logits", lg.data_ptr(), rows, 1.0, None, ids.data_ptr(), w.data_ptr(), st())
+    p = torch.softmax(lg.double(), -1)
+    ref = torch.sort(p, dim=-1, descending=True, stable=True)
+    assert torch.equal(ids[:-1], ref.indices[:-1, :6]) and ids[-1].tolist() == list(range(6))
+    assert rel_err(w, p.gather(1, ids)) < 1e-6
