@@ -121,7 +121,7 @@ def time_dominant_kernel(eng, family: str, reps: int = 4) -> dict:
             call("dsv2_moe_route_gateup", ptr(b.xn), B, ptr(b.ids32), ptr(L.w_gu), ptr(L.sh_gu), c.moe_inter,
                  ptr(b.hbuf), stream_ptr())
     elif eng.expert_dtype == "fp8":
-        sym = {32: "gemm_f8_kernel<true, 16, 4>", 64: "gemm_f8_kernel<true, 32, 4>"}[b.tile_tokens]
+        sym = {32: "gemm_f8_kernel<true, 16, 128, 3, 3>", 64: "gemm_f8_kernel<true, 32, 64, 8, 4>"}[b.tile_tokens]
         n_exp = int(torch.unique(b.ids32[:B]).numel())
         # e4m3 weights (1 B) + one fp32 scale per weight row, routed and shared; bf16 outputs
         bytes_per = (n_exp * 2 * c.moe_inter + 2 * c.shared_inter) * (c.hidden + 4) + (B * 6 * c.moe_inter
@@ -137,8 +137,8 @@ def time_dominant_kernel(eng, family: str, reps: int = 4) -> dict:
         from dsv2lite.engine import shared_in_grouped
 
         sym = {16: "gemm_xlds_kernel<1, true, 4, true, 2, 2, 1, false>",
-               32: "gemm_xlds_kernel<2, true, 4, true, 2, 4, 2, true>", 64: "gemm_dma_kernel<true, 32, 32, 4, 2>",
-               256: "gemm_dma_kernel<true, 64, 128, 2, 4>"}[b.tile_tokens]
+               32: "gemm_xlds_kernel<2, true, 4, true, 2, 4, 2, true>", 64: "gemm_dma_kernel<true>",
+               256: "gemm_big_kernel<true>"}[b.tile_tokens]
         n_exp = int(torch.unique(b.ids32[:B]).numel())
         bytes_per = n_exp * 2 * c.moe_inter * c.hidden * 2 + B * 6 * c.moe_inter * 2
         if shared_in_grouped(B, b.tile_tokens):
@@ -522,9 +522,7 @@ def bench_mla_micro(args) -> dict:
     base_d = base.to(dev)
     # the planner with 640 workgroups (5 splits of the longest row), which suits these very
     # unequal lengths (the engine's 256 suits its batches: 320 and 384 made the bsz=64 step
-    # 1.5% / 0.7% slower); measured on MI355X, decode kernel: split 1664 (5 splits) 120.3 us,
-    # 1728 117.5, 1792 119.6, 1920 121.5, 2048 (4 splits) 126.5, 2304 140.5, 1536 (6 splits)
-    # 147.6, 1280 130.3, 3072 169.3
+    # 1.5% / 0.7% slower)
     split, ns = plan_splits(B, max(lens), target_wgs=640)
     # a row goes in equal pieces of at most `split`; whole multiples of 256 tokens (1,792 here) pack
     # these lengths best: decode kernel 121.3 us, 137.3 at 1,664, 130.8 at 2,048

@@ -61,9 +61,9 @@ GEMM_ROUTER_MIN_ROWS = 1024
 # prefill chunks from this many rows bucket their routes over many workgroups (one workgroup
 # is VALU-bound there: 8192 rows 74 us, against three short launches)
 WIDE_BUCKET_MIN_ROWS = 1024
-# grouped MoE: from this many routes in a launch the 256-token tiles (256 x 256 ring GEMM, one
-# MFMA per 384 B of LDS reads) beat the 64-token ones.  The crossover follows the launch's
-# routes rather than their spread over the experts: measured on MI355X, routed gate_up + down,
+# grouped MoE: from this many routes in a launch the 256-token tiles beat the 64-token ones.  The
+# crossover follows the launch's routes rather than their spread over the experts: measured on
+# MI355X with an earlier, slower form of the large-tile kernel, routed gate_up + down,
 # uniform routing (all 64 experts) 4096 routes 297 vs 321 us (64 vs 256 tokens), 6144 routes
 # 421 vs 358 us, 49152 routes 2264 vs 1155 us; every row on the same 6 experts 3072 routes
 # 109 vs 120 us, 6144 routes 213 vs 194 us
