@@ -424,7 +424,9 @@ class DecodeEngine:
             call("dsv2_mla_prepare_qlat", ptr(b.qkva), c.qkva_dim, R, ptr(pos), ptr(base), ptr(cap),
                  ptr(L.kv_norm), c.eps, ptr(self.cos), ptr(self.sin), self.max_pos, ptr(L.w_ukt), ptr(cache),
                  ptr(b.q), ptr(self.cache.status), st)
-        if family == "batch" and b.max_splits == 1:
+        # the small family keeps o_lat in fp32 up to W_UV, whichever family's kernels run its step
+        w_uv = L.w_uv if self.family == "small" else None
+        if w_uv is None and b.max_splits == 1:
             # one split per row (~256+ rows fill the GPU): normalised o_lat straight from the decode
             call("dsv2_mla_decode_rows", ptr(b.q), ptr(cache), ptr(base), ptr(pos), ptr(cap), R, self.scale,
                  ptr(b.olat), c.n_heads * c.kv_rank, st)
@@ -435,17 +437,19 @@ class DecodeEngine:
             return
         call("dsv2_mla_decode", ptr(b.q), ptr(cache), ptr(base), ptr(pos), ptr(cap), R, b.split_tokens,
              b.max_splits, self.scale, ptr(b.part_o), ptr(b.part_ml), st)
-        if family == "small":
+        if w_uv is not None:
             call("dsv2_mla_combine", ptr(b.part_o), ptr(b.part_ml), ptr(pos), ptr(cap), R, b.split_tokens,
-                 b.max_splits, ptr(L.w_uv), ptr(b.attn), c.hidden, st)
-            call("dsv2_gemv_bf16", ptr(b.attn), c.hidden, R, c.hidden, ptr(L.w_o), c.hidden, None, 0.0, ptr(b.h),
-                 c.hidden, ptr(b.h), c.hidden, 0, st)
+                 b.max_splits, ptr(w_uv), ptr(b.attn), c.hidden, st)
         else:
             call("dsv2_mla_combine", ptr(b.part_o), ptr(b.part_ml), ptr(pos), ptr(cap), R, b.split_tokens,
                  b.max_splits, None, ptr(b.olat), c.n_heads * c.kv_rank, st)
             # attn[r, h*128 + i] = W_UV_h o_lat[r, h]: 16 head groups, K = 512
             call("dsv2_gemm_bf16", ptr(b.olat), c.n_heads * c.kv_rank, c.kv_rank, R, c.kv_rank, ptr(L.w_uv),
                  c.v_dim * c.kv_rank, c.v_dim, c.n_heads, None, 0, ptr(b.attn), c.hidden, c.v_dim, 0, st)
+        if family == "small":
+            call("dsv2_gemv_bf16", ptr(b.attn), c.hidden, R, c.hidden, ptr(L.w_o), c.hidden, None, 0.0, ptr(b.h),
+                 c.hidden, ptr(b.h), c.hidden, 0, st)
+        else:
             call("dsv2_gemm_bf16", ptr(b.attn), c.hidden, 0, R, c.hidden, ptr(L.w_o), 0, c.hidden, 1, ptr(b.h),
                  c.hidden, ptr(b.h), c.hidden, 0, 0, st)
 

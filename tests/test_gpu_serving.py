@@ -130,6 +130,38 @@ def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("rows,cap", [(4, 40), (5, 40), (8, 400), (40, 40), (40, 400)])
+def test_small_family_keeps_the_latent_output_in_fp32(rows, cap):
+    """The small family applies W_UV to the fp32 latent output at every row count.  With zero
+    queries all scores are 0, the softmax weights are exact and o_lat is the mean of the row's
+    latents, which fp32 holds almost exactly and bf16 does not: bf16(W_UV o_lat) then equals the
+    float64 result but for values next to a rounding boundary (fp32 sums of 512 terms: within
+    512 * 2^-24 of the sum of magnitudes, about 2^-11 of a bf16 step's width here), where a bf16
+    o_lat moves a large share of them."""
+    import dsv2lite
+
+    cfg = dsv2lite.DSV2Config(n_layers=1)
+    w = dsv2lite.init_weights(cfg, device="cuda", seed=0)
+    L = w.layers[0]
+    L.w_qkva[:cfg.n_heads * (cfg.qk_nope + cfg.qk_rope)].zero_()
+    eng = dsv2lite.DecodeEngine(w, [cap] * rows, family="small")
+    lens = [3 + (7 * i) % (cap - 8) for i in range(rows)]
+    eng.prefill(_prompts(lens, 12))
+    eng.step()
+    torch.cuda.synchronize()
+    eng.check_errors()
+    cache, w_uv = eng.cache.layer(0), L.w_uv.double().reshape(cfg.n_heads * cfg.v_dim, cfg.kv_rank)
+    differ = total = 0
+    for b, n in enumerate(lens):
+        base = int(eng.cache.base[b])
+        olat = cache[base:base + n + 1, :cfg.kv_rank].double().mean(0)
+        want = (w_uv @ olat).to(torch.bfloat16)
+        differ += int((eng.buf.attn[b] != want).sum())
+        total += want.numel()
+    print(f"{rows} rows, capacity {cap}: {differ} of {total} differ from bf16 of the float64 result", flush=True)
+    assert differ <= 0.02 * total
+
+
 def test_small_family_absorb_and_split_decode_agree_at_the_threshold(weights):
     """The small family's attention just below and above the capacity at which "absorb" hands over
     to the split-KV decode: same prompt, logits within the 2e-2 parity bar of each other."""
