@@ -340,10 +340,9 @@ class DecodeEngine:
             self.buf.set_tile_tokens(self._fit_tile(moe_tile))
             self._moe_tiles_tuned = True
         elif self.step_family == "batch":
+            # the small family keeps this tile whatever its rows route to, so a row's results do not
+            # depend on the batch it was captured with
             self.buf.set_tile_tokens(self._fit_tile(self.buf.tile_tokens))
-            # a few rows of the small family keep this tile whatever they route to, so a row's
-            # results do not depend on the batch it was captured with
-            self._moe_tiles_tuned = family == "small" and self.B <= 16
         self._amax = torch.empty(max(0, _hip.lib.dsv2_lm_head_argmax_workspace_size(min(self.B, 8))),
                                  dtype=torch.uint8, device=device)
         # small family: one fused workgroup per (row, head) while contexts are short; the
@@ -757,7 +756,7 @@ class DecodeEngine:
         (state restored afterwards), like the reference's tile selection before capture
         (moe_batch.py:596-657) but without timing runs: the median over MoE layers of
         routing_load, mapped by tile_tokens_for_load.  Returns the tile."""
-        if self.step_family != "batch":
+        if self.family != "batch":
             return 0
         snap = self.snapshot()
         rec: list = []
@@ -776,7 +775,7 @@ class DecodeEngine:
         family first picks its MoE token tile from one eager step (tune_moe_tiles).  Sets
         kernels_per_step to the number of nodes of the captured graph (every node is a kernel
         launch: the step records no copies or memsets)."""
-        if self.step_family == "batch" and not getattr(self, "_moe_tiles_tuned", False):
+        if self.family == "batch" and not getattr(self, "_moe_tiles_tuned", False):
             self.tune_moe_tiles()
         saved = list(self._host_pos)
         g = torch.cuda.CUDAGraph(keep_graph=True)

@@ -103,18 +103,20 @@ def test_prefill_takes_prompts_from_host_or_device_alike(weights, where):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("rows", [4, 5, 8])
+@pytest.mark.parametrize("rows", [4, 5, 8, 17, 40])
 def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
     """The small family below and from the row count at which its step runs the batch family's
     kernels: graph replay equals the eager step bitwise, and a sequence decodes to the same bits
-    whatever prompts share its batch."""
+    whatever prompts share its batch -- prompts that spread over the experts (two sets of them) or
+    one repeated token, whose rows all go to the same experts."""
     import dsv2lite
 
     mine = _prompts([11], 7)[0]
     got = []
-    for seed in (8, 9):
+    lens = [3 + i % 20 for i in range(rows - 1)]
+    for others in (_prompts(lens, 8), _prompts(lens, 9), [torch.full((n,), 77).cuda() for n in lens]):
         eng = dsv2lite.DecodeEngine(weights, [32] * rows, family="small")
-        eng.prefill([mine] + _prompts([3 + i for i in range(rows - 1)], seed))
+        eng.prefill([mine] + others)
         snap = eng.snapshot()
         eng.step()
         eager = eng.logits.clone()
@@ -127,7 +129,7 @@ def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
                 assert torch.equal(eng.logits, eager)
         eng.check_errors()
         got.append(eng.logits[0].clone())
-    assert torch.equal(*got)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
 @pytest.mark.parametrize("rows,cap", [(4, 40), (5, 40), (8, 400), (40, 40), (40, 400)])
