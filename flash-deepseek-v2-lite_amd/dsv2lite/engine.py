@@ -304,9 +304,10 @@ class DecodeEngine:
     def __init__(self, weights: ModelWeights, capacities: list[int], family: str = "small",
                  max_prefill_rows: int = 8192, device="cuda", mla_path: str = "absorb", moe_tile: int | None = None,
                  expert_dtype: str = "bf16"):
-        """capacities: cache tokens of each row (slot).  moe_tile (batch family): fix the
-        grouped MoE token tile (16, 32, 64 or 256) instead of choosing it from the routing of one
-        eager step at capture -- for a serving loop whose batch changes under one graph.
+        """capacities: cache tokens of each row (slot).  moe_tile (a step on the batch family's
+        kernels): fix the grouped MoE token tile (16, 32, 64 or 256) instead of choosing it from the
+        routing of one eager step at capture (small family: from the row count) -- for a serving
+        loop whose batch changes under one graph.
         expert_dtype "fp8": the decode step reads the e4m3 expert weights of
         quantize_experts_fp8 (small family: the route kernels; batch family: the grouped
         launches, 32- or 64-token tiles); prefill keeps the bf16 kernels on the dequantized
@@ -336,7 +337,7 @@ class DecodeEngine:
         self.ids = torch.zeros(self.B, dtype=torch.int64, device=device)
         self.logits = torch.empty(self.B, cfg.vocab, dtype=torch.float32, device=device)
         self.buf = RowBuffers(cfg, self.B, self.step_family, self.max_pos, device)
-        if family == "batch" and moe_tile is not None:
+        if self.step_family == "batch" and moe_tile is not None:
             self.buf.set_tile_tokens(self._fit_tile(moe_tile))
             self._moe_tiles_tuned = True
         elif self.step_family == "batch":

@@ -132,6 +132,24 @@ def test_small_family_rows_do_not_depend_on_their_batch(weights, rows):
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("family,rows", [("batch", 3), ("small", 5), ("small", 24)])
+def test_moe_tile_is_honoured_on_every_batch_kernel_step(weights, family, rows):
+    """moe_tile fixes the grouped tile of any engine whose step runs the batch family's kernels,
+    through capture and replay; a tile the launches do not have is refused."""
+    import dsv2lite
+
+    for tile in (16, 32, 64, 256):
+        eng = dsv2lite.DecodeEngine(weights, [32] * rows, family=family, moe_tile=tile)
+        eng.prefill(_prompts([4 + i % 9 for i in range(rows)], 21))
+        eng.capture()
+        eng.replay()
+        torch.cuda.synchronize()
+        assert eng.buf.tile_tokens == tile
+        assert torch.isfinite(eng.logits).all()
+    with pytest.raises(ValueError, match="tile_tokens"):
+        dsv2lite.DecodeEngine(weights, [32] * rows, family=family, moe_tile=48)
+
+
 @pytest.mark.parametrize("rows,cap", [(4, 40), (5, 40), (8, 400), (40, 40), (40, 400)])
 def test_small_family_keeps_the_latent_output_in_fp32(rows, cap):
     """The small family applies W_UV to the fp32 latent output at every row count.  With zero
