@@ -63,8 +63,9 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
   if (q0 >= max(tl.y, 1)) return;
   // every index derived from the tile table is clamped into the buffers the host described
   // (a malformed table gives wrong numbers, never an access outside them)
-  const int r0 = min(max(tl.x, 0) + q0, rows - 1), nr = min(max(tl.y, 1) - q0, min(kWgQ, rows - r0)),
-            p0 = max(tl.z, 0) + q0;
+  // (clamped before q0 is added: no table value overflows an int; a position is below cache_rows)
+  const int r0 = min(min(max(tl.x, 0), rows - 1) + q0, rows - 1), nr = min(max(tl.y, 1) - q0, min(kWgQ, rows - r0)),
+            p0 = (int)min((int64_t)max(tl.z, 0), cache_rows) + q0;
   const int64_t sb = tl.w;  // cache row of position 0 of the tile's sequence
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, kg = lane >> 4;
   int jq[kQB], qp[kQB];

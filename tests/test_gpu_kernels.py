@@ -1245,6 +1245,31 @@ def test_mla_prefill_query_tile_sizes_agree_bitwise(lens):
         at += n
 
 
+@pytest.mark.parametrize("halves", [True, False])
+def test_mla_prefill_malformed_tile_table_stays_inside(halves):
+    """Tile entries with values at the ends of int32, beside valid ones: rows and positions are
+    clamped into the buffers before a half tile's offset is added, so nothing past the output's rows
+    is written and the rows the malformed entries do not name keep their results."""
+    n, guard = 200, 256
+    top = 2 ** 31 - 1
+    bad = [(top, 128, 0, 0), (top - 63, 100, top, -5), (top, top, top - 64, top), (-7, -3, -9, -top), (n - 1, top, top, n)]
+    good = [(128, 72, 128, 0), (0, 128, 0, 0)]
+    cache, ke, ve = rnd(n, 576, seed=240), rnd(n, 16, 128, seed=241), rnd(n, 16, 128, seed=242)
+    qkva, qrope = rnd(n, 3648, seed=243), rnd(n, 16, 576, seed=244)
+    outs = []
+    for tiles in (good, bad + good):
+        tiles = tiles + [good[0]] * (2 if halves else 32)
+        assert (len(tiles) < 32) == halves
+        td = torch.tensor(tiles, dtype=torch.int32, device=DEV)
+        out = torch.full((n + guard, 2048), -3.0, dtype=BF, device=DEV)
+        call("dsv2_mla_prefill_attention", qkva.data_ptr(), 3648, qrope.data_ptr(), 16 * 576, n, cache.data_ptr(), n,
+             ke.data_ptr(), ve.data_ptr(), 0, n, td.data_ptr(), len(tiles), 0.1147, out.data_ptr(), 2048, st())
+        torch.cuda.synchronize()
+        assert torch.all(out[n:] == -3.0)
+        outs.append(out)
+    assert torch.equal(outs[0][1:n - 1], outs[1][1:n - 1])
+
+
 @pytest.mark.parametrize("split,lens", [(32, [1, 32, 33, 64, 65, 97]), (96, [95, 96, 97, 193, 289, 300]),
                                         (160, [161, 320, 321, 479, 480, 500])])
 def test_mla_decode_equal_pieces(split, lens):
