@@ -757,7 +757,11 @@ __device__ __forceinline__ void big_tload(const BigSrc& s, uint8_t* lds, int j, 
 
 // The accumulators stay in the 256 AGPRs of a lone wave per SIMD (as a builtin the compiler copies
 // them to and from VGPRs between the MFMAs, and spills).  The hazards the compiler would cover are
-// met by hand: nothing but these MFMAs touches an accumulator between the two s_nop fences.
+// met by hand: nothing but these MFMAs touches an accumulator between the two s_nop fences.  What
+// the compiler could still place there -- the zeroes, a copy of an accumulator, a VALU write of a
+// fragment -- the build looks for in the assembly and refuses (build.py, mfma_hazards); tying the
+// fences to the accumulators by operands instead costs 72 to 88 spilled registers for 26 to 32
+// (MI355X, routed experts of 4,001 tokens 583 -> 637 us).
 __device__ __forceinline__ void mfma_acc(floatx4_t& c, const bf16x8_t& a, const bf16x8_t& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }

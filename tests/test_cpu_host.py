@@ -405,3 +405,40 @@ def test_chunk_segments_equal_the_rows_own_runs():
     for s in range(sum(lens)):
         for e in range(s + 1, sum(lens) + 1):
             assert _chunk_segments(lens, s, e) == _segments(seq[s:e], posv[s:e])
+
+
+def _mfma_hazards():
+    import importlib.util
+    import os
+
+    import triton_kernels
+
+    path = os.path.join(os.path.dirname(os.path.dirname(triton_kernels.__file__)), "csrc", "build.py")
+    spec = importlib.util.spec_from_file_location("dsv2_build", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod.mfma_hazards
+
+
+@pytest.mark.parametrize("body,n", [
+    # the accumulator read behind its fence, the fragment from LDS: fine
+    ("ds_read_b128 v[4:7], v1\n s_waitcnt lgkmcnt(0)\n MFMA\n s_nop 15\n s_nop 15\n v_accvgpr_read_b32 v9, a0", 0),
+    ("v_accvgpr_write_b32 a0, 0\n s_nop 15\n MFMA\n v_add_u32_e32 v20, v21, v22\n s_nop 15\n s_nop 1\n "
+     "v_accvgpr_read_b32 v9, a0", 0),
+    # an accumulator copied right behind its MFMA, written right before it
+    ("MFMA\n v_accvgpr_read_b32 v9, a0", 1),
+    ("MFMA\n s_nop 15\n v_accvgpr_mov_b32 a8, a0", 1),
+    ("v_accvgpr_write_b32 a3, v2\n MFMA", 1),
+    # a fragment moved in front of the MFMA that reads it
+    ("v_mov_b32_e32 v5, v30\n s_nop 0\n MFMA", 1),
+    ("v_mov_b32_e32 v5, v30\n s_nop 1\n MFMA", 0),
+    # over a loop's back edge: the MFMA ends the body, the access starts it
+    (".LBB0_1:\n v_accvgpr_read_b32 v9, a0\n s_nop 15\n s_nop 15\n MFMA\n s_cbranch_scc1 .LBB0_1", 1),
+])
+def test_build_finds_mfma_hazards_in_inline_asm(body, n):
+    """The build's check of the large-tile GEMM's assembly: wait states before anything else touches
+    an accumulator and after a VALU write of a source, along the code and over branches."""
+    mfma = "v_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]"
+    asm = f"_Z9my_kernelv: ; @_Z9my_kernelv\n{body.replace('MFMA', mfma)}\n s_endpgm\n.Lfunc_end0:\n"
+    assert len(_mfma_hazards()(asm, "my_kernel")) == n
+    assert _mfma_hazards()(asm, "other_kernel")  # a kernel the check no longer finds is a failure too
