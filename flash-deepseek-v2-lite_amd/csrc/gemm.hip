@@ -439,6 +439,7 @@ constexpr int kDmaGroupedWgs = 512;  // 256 CUs x 2 (64 KB of LDS each)
 
 struct DmaShape {
   int tiles, nwg, nfb;
+  bool rotate;  // work items start at different K chunks
 };
 
 // SWIGLU: the 64 weight rows of a workgroup are, per 16 features, 16 gate rows then the 16
@@ -529,15 +530,16 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const GemmArgs a, const D
       }
       dst[j] = (tok ? TM * RB + ((TN / NW) * wv + RPL * (j - LW)) * RB : ((TM / NW) * wv + RPL * j) * RB);
     }
-    // grouped: the item's K chunks start at a rotation that spreads the workgroups' concurrent
-    // requests over the weight rows' address range instead of one column of 128 B lines (C3
-    // grouped gate_up 158.4 -> 153.6 us).  It depends on (expert or shared half, feature block)
-    // only: an expert's results do not depend on which other tiles share the launch, and the
-    // token tiles of one weight block read its chunks in the same order, so the ones that run
-    // together share each chunk's fetch in L2 (a rotation per token tile as well made the
-    // reference workload at bsz=256 -- 4 tiles per expert -- 1.5x slower).  Dense launches take
-    // their chunks in order: each output then is the same sum, bit for bit, as gemm_big_kernel's
-    const int rot = a.tiles ? (int)((unsigned)(fb * 7 + g * 13 + (shared ? 3 : 0)) % (unsigned)nch) : 0;
+    // rotate (grouped, and dense weights of tens of MB): the item's K chunks start at a rotation
+    // that spreads the workgroups' concurrent requests over the weight rows' address range instead
+    // of one column of 128 B lines (C3 grouped gate_up 158.4 -> 153.6 us; lm_head at 33 rows 93 ->
+    // 86, dense layer-0 gate_up at 33 rows 26.7 -> 22.9; qkv_a and smaller weights the same or a
+    // little slower).  It depends on (expert or shared half, feature block) only: an expert's
+    // results do not depend on which other tiles share the launch, and the token tiles of one
+    // weight block read its chunks in the same order, so the ones that run together share each
+    // chunk's fetch in L2 (a rotation per token tile as well made the reference workload at
+    // bsz=256 -- 4 tiles per expert -- 1.5x slower)
+    const int rot = sh.rotate ? (int)((unsigned)(fb * 7 + g * 13 + (shared ? 3 : 0)) % (unsigned)nch) : 0;
     auto issue = [&](int chunk, int buf) {
       int cc = min(chunk, nch - 1) + rot;  // past the last chunk: repeat it (never multiplied)
       if (cc >= nch) cc -= nch;
@@ -640,8 +642,12 @@ __global__ __launch_bounds__(256) void gemm_dma_kernel(const GemmArgs a, const D
 }
 
 // grouped: max_tiles entries of a table of 64-token tiles; dense: a.rows tokens
+// dense weights that stream from HBM whole while few token tiles read them (lm_head, dense gate_up)
+static bool wide_weights(int N, bool swiglu) { return N >= (swiglu ? 8192 : 16384); }
+
 static void launch_dma(const GemmArgs& a, bool swiglu, hipStream_t st, int max_tiles = 0) {
   DmaShape sh;
+  sh.rotate = a.tiles || wide_weights(a.N, swiglu);
   // plain: a last feature block past N (N % 64 == 0) repeats row N-1 and stores nothing there
   sh.nfb = swiglu ? a.N / 32 : (a.N + 63) / 64;
   sh.tiles = a.tiles ? max_tiles : (a.rows + 63) / 64;
@@ -1523,26 +1529,29 @@ static int pick_tb(int rows) { return rows <= 16 ? 1 : (rows <= 32 ? 2 : (rows <
 // features x 2048: 128 rows 20.0 -> 11.3 us; 10944: 42 -> 24.6), many features (3648: 13.8 ->
 // 11.6) and else 160 (2048 x 2048: 211 rows, 128 items, 10.4 against 11.5 us; 300 rows, 160
 // items, 14.8 -> 11.6; K = 10944: 300 rows 61 -> 42); the lm_head (102400 x 2048) and the dense
-// layer's gate_up (SwiGLU, 10944 x 2048) from 33 rows (64 rows: 116 -> 100 and 35.6 -> 28.8).
-// Ring or large tiles: the cheaper by their measured times (us; K = 2048, 2816, 10944 at 512 to
-// 8192 rows, within about 15% of each).  The ring takes 4 + 0.034 per item and 2048 of K (512
-// items resident); the large tiles 8 + per round of 256 items K / 64 chunks of 0.75 / 0.82 / 0.95
-// / 1.2 us for 64 / 128 / 192 / 256 tokens and 3 between rounds.  E.g. 1149 rows x 2048 x 2048:
-// ring 24.8, large 29.8 / 33.6 / 38.8 / 47.2; 2300 rows x 3648: 73 against 77 / 62 / 42 / 50;
-// 8192 rows x 10944 (SwiGLU): 1525 against 637 with 256 tokens; lm_head at 200 rows 199 -> 141.
+// layer's gate_up (SwiGLU, 10944 x 2048) from 33 rows (64 rows: 116 -> 99 and 35.6 -> 25.7).
+// Ring or large tiles: the cheaper by their measured times (us).  The ring takes 4 + 0.034 per item
+// and 2048 of K (512 items resident); the large tiles 8 + per round of 256 items K / 64 chunks of
+// 0.75 / 0.82 / 0.95 / 1.2 us for 64 / 128 / 192 / 256 tokens and 3 between rounds, and 0.15 per MB
+// of weights and tokens: their one workgroup per CU has two chunks in flight, which does not cover
+// operands that come from HBM.  Where the lines fall, ring against the best large tiles: lm_head
+// 100 rows 123 / 130, 129 rows 155 / 136; gate_up 10944 at 129 rows 39.4 / 45.3, 192 rows 43.4 /
+// 45.8, 256 rows 53.5 / 48.6; 2048 x 10944 at 1,500 rows 130 / 184, 2,047 rows 198 / 185; 3648 x
+// 2048 at 1,500 rows 44 / 35; 8192 rows x 10944 (SwiGLU) 1525 / 637.
 static int dense_tiles(int rows, int N, int K, bool swiglu) {
   if (swiglu ? N % 32 != 0 : N % 64 != 0) return -1;
   const int64_t items = (int64_t)((rows + 63) / 64) * (swiglu ? N / 32 : N / 64);
-  const bool wide = rows > 32 && N >= (swiglu ? 8192 : 16384);
+  const bool wide = rows > 32 && wide_weights(N, swiglu);
   if (!wide && (rows <= 64 || items < (swiglu ? 128 : (N >= 3072 ? 100 : 160)))) return -1;
   const double ring_us = 4.0 + K / 2048.0 * (0.034 * items > 8.0 ? 0.034 * items : 8.0);
   const double chunk_us[4] = {0.75, 0.82, 0.95, 1.2};
+  const double stream_us = 0.15e-6 * 2.0 * K * ((double)N * (swiglu ? 2 : 1) + rows);
   int best = 0;
   double best_us = ring_us;
   const int rows_wg = swiglu ? kBigRows / 2 : kBigRows;
   for (int ng = 1; ng <= 4; ++ng) {
     const int64_t n = (int64_t)((rows + 64 * ng - 1) / (64 * ng)) * ((N + rows_wg - 1) / rows_wg);
-    const double us = 5.0 + (double)((n + kBigWgs - 1) / kBigWgs) * (3.0 + K / 64 * chunk_us[ng - 1]);
+    const double us = 5.0 + stream_us + (double)((n + kBigWgs - 1) / kBigWgs) * (3.0 + K / 64 * chunk_us[ng - 1]);
     if (us < best_us) {
       best_us = us;
       best = ng;
@@ -1662,6 +1671,10 @@ extern "C" int dsv2_gemm_bf16(const void* x, int64_t x_stride, int64_t x_gstride
   const int64_t grid_y = (int64_t)a.tiles_per_group * n_groups;
   DSV2_REQUIRE(grid_y <= 65535, DSV2_E_SHAPE, "gemm: too many row tiles (%lld)", (long long)grid_y);
   return launch_gemm(a, tb, swiglu, (int)grid_y, (hipStream_t)stream);
+}
+
+extern "C" int dsv2_gemm_dense_tiles(int rows, int K, int N, int flags) {
+  return dense_tiles(rows, N, K, flags & DSV2_LINEAR_SWIGLU);
 }
 
 // ---------------------------------------------------------------------------

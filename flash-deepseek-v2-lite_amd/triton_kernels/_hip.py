@@ -73,6 +73,7 @@ _SIGS = {
     "dsv2_moe_route_gateup_i64": ([_p, _i32, _p, _p, _p, _i32, _p, _p], _i32),
     "dsv2_moe_route_down": ([_p, _i32, _p, _p, _p, _p, _i32, _i32, _p, _p, _p, _p], _i32),
     "dsv2_moe_route_down_i64": ([_p, _i32, _p, _p, _p, _p, _i32, _i32, _p, _p, _p, _p], _i32),
+    "dsv2_gemm_dense_tiles": ([_i32, _i32, _i32, _i32], _i32),
     "dsv2_moe_bucket": ([_p, _i32, _i32, _p, _p, _p, _p, _p], _i32),
     "dsv2_moe_bucket_i64": ([_p, _i32, _i32, _p, _p, _p, _p, _p], _i32),
     "dsv2_moe_bucket_workspace_size": ([_i32], _i64),

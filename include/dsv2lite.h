@@ -150,6 +150,11 @@ int dsv2_gemm_bf16(const void* x, int64_t x_stride, int64_t x_gstride, int rows,
                    int64_t w_gstride, int N, int n_groups, const void* residual, int64_t res_stride, void* y,
                    int64_t y_stride, int64_t y_gstride, int flags, void* stream);
 
+/* The tile shape dsv2_gemm_bf16 takes for one group of that size (flags: DSV2_LINEAR_SWIGLU counts):
+ * 0 the 64-feature x 64-token ring, 1..4 the 256-row large tiles of 64 n tokens, -1 another kernel.
+ * Host arithmetic only. */
+int dsv2_gemm_dense_tiles(int rows, int K, int N, int flags);
+
 /* ---- absorbed MLA -------------------------------------------------------- */
 
 /* Per-row cache bounds (every MLA entry point): row r owns cache rows

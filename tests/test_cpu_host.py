@@ -442,3 +442,19 @@ def test_build_finds_mfma_hazards_in_inline_asm(body, n):
     asm = f"_Z9my_kernelv: ; @_Z9my_kernelv\n{body.replace('MFMA', mfma)}\n s_endpgm\n.Lfunc_end0:\n"
     assert len(_mfma_hazards()(asm, "my_kernel")) == n
     assert _mfma_hazards()(asm, "other_kernel")  # a kernel the check no longer finds is a failure too
+
+
+@pytest.mark.parametrize("K,N,swiglu,rows,tiles", [
+    # (first rows, last rows) of each choice measured on MI355X for the model's dense products:
+    # lm_head, the dense layer's gate_up and down, q|kv_a
+    (2048, 102400, False, (33, 128), {0}), (2048, 102400, False, (129, 192), {3}), (2048, 102400, False, (193, 256), {4}),
+    (2048, 10944, True, (33, 192), {0}), (2048, 10944, True, (200, 256), {2}), (2048, 10944, True, (8192, 8192), {4}),
+    (10944, 2048, False, (300, 1536), {0}), (10944, 2048, False, (1900, 2048), {1}), (10944, 2048, False, (8192, 8192), {4}),
+    (2048, 3648, False, (65, 768), {0}), (2048, 3648, False, (1500, 1500), {2}),
+    (2048, 2048, False, (65, 256), {-1}), (2048, 2048, False, (257, 1500), {0}),
+])
+def test_dense_gemm_tile_choice(K, N, swiglu, rows, tiles):
+    from triton_kernels import _hip
+
+    for r in {rows[0], (rows[0] + rows[1]) // 2, rows[1]}:
+        assert _hip.lib.dsv2_gemm_dense_tiles(r, K, N, 1 if swiglu else 0) in tiles, r
