@@ -54,6 +54,10 @@ def pack_attention_weights(attn: torch.nn.Module) -> AttentionPackedWeights:
 ONE_SPLIT_MAX_CTX = 256
 
 
+# one split per row also up to this cache length where rows alone leave under a third of the CUs idle
+IDLE_CU_ONE_SPLIT_CTX = 512
+
+
 def plan_splits(rows: int, max_ctx: int, target_wgs: int = 256) -> tuple[int, int]:
     """(split_tokens, max_splits) for the split-KV decode: one split per row for caches of at
     most ONE_SPLIT_MAX_CTX tokens (measured on MI355X, whole decode steps, against the
@@ -61,18 +65,24 @@ def plan_splits(rows: int, max_ctx: int, target_wgs: int = 256) -> tuple[int, in
     6.901, bsz=128 x 233 7.941 -> 7.832; at 433 tokens one split loses, 7.013 -> 7.101);
     else the most splits per row (at most 64, split_tokens a multiple of 32) that leave at most
     target_wgs workgroups: 256 = one per CU, each streaming its split with two tiles in flight.
-    A few more than 256 make some CUs run two while the rest run one: attention calls of 96 rows
-    x 3,301 tokens 119.8 us with 288, 106.5 with 192, 107.8 with 384; 40 x 6,001 97.5 with 280,
-    90.9 with 200; 70 x 1,601 72.6 with 280, 64.3 with 210.  Where that leaves one split per row
-    and under 171 rows, three (two workgroups on most CUs): 140 rows x 1,601 tokens 108 -> 95 us,
-    160 108 -> 101, but 180 109 -> 119.  Rows of very unequal lengths want more, shorter splits
-    (bsz=128 x U[256,8192]: 512 -> 2048-token splits 132 us, 256 -> 4064-token splits 171 us);
-    capping the split at 2048 tokens instead cost the equal-length bsz=256 step 8%."""
+    A few more than 256 make some CUs run two while the rest run one (70 rows x 1,600 tokens 39
+    us with 4, 33 with 3; 40 x 4,096 52 with 7, 40 with 6).  Where that leaves one or two splits per
+    row and CUs idle, a long row among short ones would end the launch alone, so there are more:
+      under 128 rows, two workgroups per CU (decode + merge of 96 rows x 3,300 tokens, 2 / 3 / 5
+      splits: equal lengths 72 / 82 / 69 us, lengths from an eighth 64 / 61 / 51, one full row among
+      sixteenths 62 / 45 / 31; 110 x 2,048 with 2 / 3 / 4: 50 / 60 / 54, 45 / 47 / 41, 43 / 32 / 27);
+      under 171, three (140 x 1,600: 57 us, 66 with 2);
+      under 256, two past IDLE_CU_ONE_SPLIT_CTX tokens (200 x 2,048, 1 / 2 / 3 splits: 86 / 89 / 101,
+      72 / 68 / 75, 69 / 46 / 39; but 200 x 512 25 / 34 / 40, 23 / 30 / 31, 21 / 20 / 21).
+    More than that suits lengths spread as wide as 128 rows of U[256,8192] (1,664-token splits 126
+    us, 4,096-token ones 150), which a caller plans with a larger target_wgs."""
     if max_ctx <= ONE_SPLIT_MAX_CTX:
         return max(32, math.ceil(max_ctx / 32) * 32), 1
     per_row = max(1, min(64, target_wgs // max(rows, 1)))
-    if per_row == 1 and target_wgs // 2 < rows and 3 * rows <= 2 * target_wgs:
-        per_row = 3
+    if per_row == 2 and 2 * rows < target_wgs:
+        per_row = 2 * target_wgs // rows
+    elif per_row == 1 and rows < target_wgs:
+        per_row = 3 if 3 * rows <= 2 * target_wgs else (2 if max_ctx > IDLE_CU_ONE_SPLIT_CTX else 1)
     split = max(32, math.ceil(math.ceil(max_ctx / per_row) / 32) * 32)
     split = max(split, math.ceil(max_ctx / 64 / 32) * 32)
     return split, math.ceil(max_ctx / split)

@@ -94,6 +94,21 @@ def test_plan_splits(rows, ctx):
         assert ns == 1
 
 
+@pytest.mark.parametrize("rows,ctx,ns", [
+    (64, 1024, 4), (70, 1600, 3), (85, 3300, 3), (86, 3300, 5), (96, 3300, 5), (103, 2048, 4), (127, 4096, 4),
+    (128, 4096, 2), (140, 1600, 3), (170, 2048, 3), (171, 2048, 2), (200, 2112, 2), (255, 4096, 2), (200, 512, 1),
+    (255, 512, 1), (256, 2048, 1)])
+def test_plan_splits_leaves_no_long_row_alone(rows, ctx, ns):
+    """With CUs to spare a row's tokens go to several workgroups, so one long row among short ones
+    does not end the launch alone: at least as many splits as ceil(256 / rows) from 86 rows, but for
+    caches up to 512 tokens, where the merge costs more."""
+    from dsv2lite.engine import plan_splits
+
+    assert plan_splits(rows, ctx)[1] == ns
+    if rows > 85 and ctx > 512:
+        assert ns >= math.ceil(256 / rows)
+
+
 def test_moe_tile_choice_and_cache_layout():
     from dsv2lite.cache import CompressedKVCache
     from dsv2lite.engine import moe_tile_tokens
