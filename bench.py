@@ -524,10 +524,6 @@ def bench_mla_micro(args) -> dict:
     # unequal lengths (the engine's 256 suits its batches: 320 and 384 made the bsz=64 step
     # 1.5% / 0.7% slower)
     split, ns = plan_splits(B, max(lens), target_wgs=640)
-    # a row goes in equal pieces of at most `split`; whole multiples of 256 tokens (1,792 here) pack
-    # these lengths best: decode kernel 121.3 us, 137.3 at 1,664, 130.8 at 2,048
-    split = -(-split // 256) * 256
-    ns = math.ceil(max(lens) / split)
     if args.mla_split:
         split, ns = args.mla_split, math.ceil(max(lens) / args.mla_split)
     po = torch.empty(B, ns, 16, 512, device=dev)

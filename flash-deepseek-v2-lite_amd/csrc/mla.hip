@@ -18,6 +18,7 @@ constexpr int kLat = 512;       // latent part
 constexpr int kQkvA = 3648;     // q (16*192) | latent (512) | k_pe (64)
 constexpr int kTile = 32;       // tokens per LDS tile
 constexpr int kLdsRow = kRow + 8;  // padded LDS row (elements): 1168 bytes
+constexpr unsigned kEqualPieceWgs = 480;  // decode workgroups, of the 512 resident at once (two per CU)
 }  // namespace
 
 // Workgroup (x, y) handles rows y*RB .. y*RB+RB-1.  With w_ukt != null workgroups x < 128
@@ -187,12 +188,17 @@ __global__ __launch_bounds__(256, 2) void mla_decode_kernel(const bf16_t* __rest
   const int pb = pos[b], cb = cap[b];
   const int64_t bb = base[b];
   const int len = min(pb + 1, cb);  // never past the row's own slots
-  // a row longer than split_tokens goes in ceil(len / split_tokens) pieces of equal whole tiles
-  // (pieces of split_tokens and a short rest leave the launch waiting for the full ones; MI355X,
-  // the attention call of 96 rows x 3,301 tokens in splits of 1,376: 128 -> 120 us)
+  // a row longer than split_tokens goes in ceil(len / split_tokens) pieces: equal ones of whole tiles
+  // while the launch's workgroups are all resident with CU slots to spare, since a launch that waits
+  // for full pieces while short rests are done wastes them (MI355X, decode + merge, full against equal
+  // pieces: 172 rows of 256..2,048 tokens in two 68.1 / 62.4 us, 86 x 250..2,000 in five 37.5 / 36.3);
+  // full ones and a rest beyond that, where rests fill the gaps (128 rows of U[256,8192] in pieces of
+  // 1,664: 126 us, 142 in equal ones; 255 x 2,048..4,096 in two: 166, 170)
   const int ns = len > split_tokens ? (len - 1) / split_tokens + 1 : 1;
   // (ns - 1) * piece <= (ns - 1) * split_tokens < len: none of the ns pieces is empty
-  const int piece = ns == 1 || ns > max_splits ? split_tokens : ((len + kTile - 1) / kTile + ns - 1) / ns * kTile;
+  const int piece = ns == 1 || ns > max_splits || gridDim.x * gridDim.y > kEqualPieceWgs
+                        ? split_tokens
+                        : ((len + kTile - 1) / kTile + ns - 1) / ns * kTile;
   const int t_begin = s * piece;
   if (t_begin >= len) {
     if (DIRECT) {  // a row with no cached token (capacity 0): zeros, as the combine writes

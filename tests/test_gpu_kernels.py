@@ -1293,6 +1293,29 @@ def test_mla_decode_equal_pieces(split, lens):
     assert rel_err(outs[0].float(), outs[1].float()) < 2 ** -7
 
 
+@pytest.mark.parametrize("rows,splits", [(30, 16), (31, 16), (120, 4), (121, 4), (240, 2), (241, 2)])
+def test_mla_decode_pieces_by_the_size_of_the_launch(rows, splits):
+    """Up to 480 workgroups a row's pieces are equal, above them full: with zero queries each split's
+    sum of softmax weights is the number of tokens it attended, exactly."""
+    split, cap = 128, 128 * splits
+    lens = [1 + (37 * i) % cap for i in range(rows)]
+    q, cache = torch.zeros(rows, 16, 576, dtype=BF, device=DEV), rnd(rows * cap, 576, seed=250)
+    base = torch.arange(rows, device=DEV) * cap
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    capd = torch.full((rows,), cap, dtype=torch.int32, device=DEV)
+    part_o = torch.empty(rows, splits, 16, 512, device=DEV)
+    part_ml = torch.empty(rows, splits, 16, 2, device=DEV)
+    P = lambda t: t.data_ptr()  # noqa: E731
+    call("dsv2_mla_decode", P(q), P(cache), P(base), P(pos), P(capd), rows, split, splits, 0.1147, P(part_o), P(part_ml),
+         st())
+    got = part_ml[:, :, 0, 1].cpu()
+    for b, n in enumerate(lens):
+        ns = -(-n // split)
+        piece = math.ceil(math.ceil(n / 32) / ns) * 32 if rows * splits <= 480 else split
+        want = [min(n, (s + 1) * piece) - s * piece for s in range(ns)]
+        assert got[b, :ns].tolist() == want, (b, n)
+
+
 @pytest.mark.parametrize("rows", [1, 1024, 1025, 4099])
 def test_topk6_from_logits_rows_per_workgroup(rows):
     """One and four rows per workgroup, a partial last workgroup: ids exact (ties to the lower
