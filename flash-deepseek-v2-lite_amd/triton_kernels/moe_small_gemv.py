@@ -11,9 +11,10 @@ from .moe_batch import (PackedRoutedExperts, _check, _ids, batched_grouped_route
                         packed_routed_moe_eager)
 
 # more tokens take the expert-grouped kernels, which read an expert's weights once for all its
-# tokens instead of once per route (MI355X, uniform routing, whole calls, route against grouped:
-# 6 tokens 94 vs 99 us, 7 108 vs 105, 8 122 vs 115, 16 235 vs 151)
-ROUTE_GEMV_MAX_TOKENS = 6
+# tokens instead of once per route (MI355X, whole calls, route against grouped: uniform routing, which
+# suits the grouped kernels least, 7 tokens 107 vs 114 us, 8 121 vs 126, 9 136 vs 128, 12 178 vs 149;
+# eight experts preferred 7 105 vs 88, 9 134 vs 101)
+ROUTE_GEMV_MAX_TOKENS = 8
 
 
 def batched_grouped_routed_moe_route_gemv(x: torch.Tensor, topk_ids: torch.Tensor, topk_weight: torch.Tensor,

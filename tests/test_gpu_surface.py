@@ -422,12 +422,13 @@ def test_expanded_attention_tile_edges(B, H, L, pos, Dq, Dv):
 
 
 @pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe", n) for n in (853, 854, 1024)]
-                         + [("batched_grouped_routed_moe_route_gemv", n) for n in (6, 7)])
-def test_grouped_moe_wrapper_tile_threshold(fn, tokens):
+                         + [("batched_grouped_routed_moe_route_gemv", n) for n in (6, 7, 8, 9)])
+def test_grouped_moe_wrapper_tile_threshold(fn, tokens, monkeypatch):
     """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds, the
-    route-local form below and above the tokens it hands on, experts unevenly loaded (one empty), against fp32 torch; three bf16 roundings (SwiGLU, expert
-    output, sum) of about 2^-9 each: 1e-2."""
-    from triton_kernels import moe_small_gemv
+    route-local form below and above the tokens it hands on (9 and more, where the grouped kernels
+    are faster under every routing measured), experts unevenly loaded (one empty), against fp32
+    torch; three bf16 roundings (SwiGLU, expert output, sum) of about 2^-9 each: 1e-2."""
+    from triton_kernels import _hip, moe_small_gemv
     from triton_kernels.moe_batch import PackedRoutedExperts
 
     I = 128
@@ -437,7 +438,10 @@ def test_grouped_moe_wrapper_tile_threshold(fn, tokens):
     logits = torch.randn(tokens, 64, generator=g) + torch.linspace(-2, 2, 64)
     logits[:, 5] = -1e9
     w, ids = torch.softmax(logits, -1).topk(6, -1)
+    calls, call = {}, _hip.call
+    monkeypatch.setattr(_hip, "call", lambda name, *a: (calls.__setitem__(name, a), call(name, *a))[1])
     out = getattr(moe_small_gemv, fn)(x, ids.to(DEV), w.to(DEV), PackedRoutedExperts(gu, dn, 2048, I, 64, 6))
+    assert ("dsv2_moe_route_gateup_i64" in calls) == (fn.endswith("route_gemv") and tokens <= 8)
     ref = torch.zeros(tokens, 2048)
     xc = c(x)
     for e in range(64):
