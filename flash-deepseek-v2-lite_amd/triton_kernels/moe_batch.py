@@ -16,10 +16,13 @@ from . import _hip
 from ._checks import require_cuda
 
 
-# from this many routes 256-token tiles (MI355X, 4,001 tokens: gate_up + down 1,182 us on 64-token
-# tiles, the whole call 1,151 -> 694), from this many rows the many-workgroup bucketing (40 us in
-# one workgroup there): the engine's own thresholds (dsv2lite.engine)
-BIG_TILE_ROUTES = 5120
+# From this many routes the 256-token tiles: from 1,280 tokens they are the faster ones under every
+# routing measured (MI355X, whole calls, 64- against 256-token tiles, us: 1,300 tokens uniform 461 / 313,
+# eight experts preferred 434 / 396; 4,001 uniform 1,151 / 569).  Fewer tokens on a few preferred experts
+# leave a 256-row launch short of tiles (860 tokens 335 / 391, 1,100 tokens 393 / 427, 1,200 409 / 417;
+# uniform 385 / 294, 421 / 308, 430 / 308).  From this many rows the many-workgroup bucketing (40 us in
+# one workgroup at 4,001).
+BIG_TILE_ROUTES = 7680
 WIDE_BUCKET_MIN_ROWS = 1024
 
 

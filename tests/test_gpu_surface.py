@@ -421,7 +421,7 @@ def test_expanded_attention_tile_edges(B, H, L, pos, Dq, Dv):
     assert rel_err(c(out), torch.softmax(s, -1) @ vd) < 4e-3
 
 
-@pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe", n) for n in (853, 854, 1024)]
+@pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe", n) for n in (853, 854, 1024, 1279, 1280)]
                          + [("batched_grouped_routed_moe_route_gemv", n) for n in (6, 7, 8, 9)])
 def test_grouped_moe_wrapper_tile_threshold(fn, tokens, monkeypatch):
     """batched_grouped_routed_moe below and above its 256-token-tile and bucketing thresholds, the
@@ -442,6 +442,8 @@ def test_grouped_moe_wrapper_tile_threshold(fn, tokens, monkeypatch):
     monkeypatch.setattr(_hip, "call", lambda name, *a: (calls.__setitem__(name, a), call(name, *a))[1])
     out = getattr(moe_small_gemv, fn)(x, ids.to(DEV), w.to(DEV), PackedRoutedExperts(gu, dn, 2048, I, 64, 6))
     assert ("dsv2_moe_route_gateup_i64" in calls) == (fn.endswith("route_gemv") and tokens <= 8)
+    if "dsv2_moe_grouped_down" in calls:  # (hsorted, tiles, num_tiles, max_tiles, tile_tokens, ...)
+        assert (calls["dsv2_moe_grouped_down"][4] == 256) == (tokens >= 1280)
     ref = torch.zeros(tokens, 2048)
     xc = c(x)
     for e in range(64):
@@ -453,7 +455,8 @@ def test_grouped_moe_wrapper_tile_threshold(fn, tokens, monkeypatch):
 
 
 @pytest.mark.parametrize("fn,tokens", [("batched_grouped_routed_moe_route_gemv", 3), ("batched_grouped_routed_moe", 1),
-                                       ("batched_grouped_routed_moe", 400), ("batched_grouped_routed_moe", 1100)])
+                                       ("batched_grouped_routed_moe", 400), ("batched_grouped_routed_moe", 1100),
+                                       ("batched_grouped_routed_moe", 1300)])
 def test_routed_moe_takes_int64_and_int32_ids_alike(fn, tokens):
     """int64 ids are read in place, others cast to int32: the same bits, out-of-range and negative
     ids (clamped) included."""
