@@ -40,10 +40,15 @@ FAMILIES = ("small", "batch")
 FUSED_MLA_MAX_CTX = 2048
 # small family, "absorb": caches up to this many tokens.  Its attention launch gives each of a
 # head's four workgroups every cached token; the split-KV decode spreads them over 64 splits and
-# costs two launches more.  Measured on MI355X, four-layer steps, absorb against split at 128 / 400
-# / 600 / 1100 / 1950 cached tokens: 1 row 260 vs 295 us, 288 vs 286, 299 vs 291, 325 vs 299, 370 vs
-# 314; 4 rows 511 vs 532, 535 vs 524, 550 vs 529, 576 vs 542, 627 vs 559
+# costs two launches more.  Measured on MI355X, four-layer steps, absorb against split at 64 / 256 /
+# 560 / 1000 / 2000 cached tokens: 1 row 252 vs 268 us, 268 vs 273, 284 vs 278, 309 vs 283, 365 vs
+# 301; 4 rows 491 vs 502, 507 vs 505, 524 vs 512, 552 vs 521, 608 vs 542
 ABSORB_MAX_CTX = 640
+# one row in a longer cache (up to FUSED_MLA_MAX_CTX): absorb while fewer tokens than this are
+# cached, split from there -- the step follows the row's length, not the room it has to grow (400
+# tokens 276 vs 275 us).  2 to 4 rows differ by 3% at most below the crossing and take the split path
+# throughout, so that a row's results do not depend on the others' lengths
+ABSORB_ROW_CTX = 384
 # small family (default MLA path): from this many rows the step runs the batch family's kernels.
 # The GEMV kernels read a routed expert's weights once per row that chose it and repeat the
 # dense dot products per row on the VALU (lm_head at 8 rows 174 us against 86 on MFMA, dense
@@ -355,11 +360,15 @@ class DecodeEngine:
         # small family, "absorb": the q|kv_a projection also forms the absorbed query in partial
         # sums (dsv2_qkva_absorb_bf16), then one attention launch (dsv2_mla_attend_parts)
         self.absorb_mla = self.step_family == "small" and self.max_pos <= ABSORB_MAX_CTX and mla_path == "absorb"
+        # one row in a longer cache: absorb below this position, split-KV from it (0: not so)
+        self.absorb_below = ABSORB_ROW_CTX if (self.step_family == "small" and mla_path == "absorb" and self.B == 1 and
+                                               ABSORB_MAX_CTX < self.max_pos <= FUSED_MLA_MAX_CTX) else 0
         # the path asked for, where the cache is short enough for the one- and two-launch paths at
         # all; "absorb" leaves caches past ABSORB_MAX_CTX to the split-KV decode as well
         self.mla_path = mla_path if family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX else "split"
         self.max_prefill_rows = max_prefill_rows
         self.graph = None
+        self._graphs: dict[bool, torch.cuda.CUDAGraph] = {}  # captured step by _absorbs()
         self.kernels_per_step = 0  # set by capture()
         self._host_pos = [0] * self.B  # host mirror of cache.pos, for capacity checks only
         self._free: set[int] = set()  # retired slots (continuous batching)
@@ -392,7 +401,7 @@ class DecodeEngine:
             call("dsv2_gemv_bf16", ptr(b.attn), c.hidden, R, c.hidden, ptr(L.w_o), c.hidden, None, 0.0, ptr(b.h),
                  c.hidden, ptr(b.h), c.hidden, 0, st)
             return
-        if family == "small" and self.absorb_mla and b is self.buf:
+        if family == "small" and self._absorbs() and b is self.buf:
             call("dsv2_qkva_absorb_bf16", ptr(b.h), c.hidden, R, ptr(L.w_qkva), ptr(L.ln_in), c.eps, ptr(L.w_uk),
                  ptr(b.qkva), c.qkva_dim, ptr(b.qlat_part), ptr(cache), ptr(base), ptr(pos), ptr(cap), st)
             call("dsv2_mla_attend_parts", ptr(b.qkva), c.qkva_dim, R, ptr(pos), ptr(base), ptr(cap), ptr(L.kv_norm),
@@ -602,6 +611,10 @@ class DecodeEngine:
                  ptr(self.logits), c.vocab, 0, LINEAR_OUT_F32, st)
         call("dsv2_argmax_f32", ptr(self.logits), B, c.vocab, ptr(self.ids), ptr(pos), st)
 
+    def _absorbs(self) -> bool:
+        """Whether the next step's attention runs the absorb path."""
+        return self.absorb_mla or self._host_pos[0] < self.absorb_below
+
     # ------------------------------------------------------------------ public
     def step(self, record: list | None = None) -> None:
         """Enqueue one decode step for all rows: reads self.ids, writes self.logits and the
@@ -775,18 +788,25 @@ class DecodeEngine:
         """Record one step() into a graph (positions/ids advance on every replay).  The batch
         family first picks its MoE token tile from one eager step (tune_moe_tiles).  Sets
         kernels_per_step to the number of nodes of the captured graph (every node is a kernel
-        launch: the step records no copies or memsets)."""
+        launch: the step records no copies or memsets).  An engine whose step changes with its row's
+        length (absorb_below) records both forms, and replay() launches the one of the position;
+        the graph returned is the present position's."""
         if self.family == "batch" and not getattr(self, "_moe_tiles_tuned", False):
             self.tune_moe_tiles()
-        saved = list(self._host_pos)
-        g = torch.cuda.CUDAGraph(keep_graph=True)
-        with torch.cuda.graph(g):
-            self.step()
-        self._host_pos = saved
-        self.kernels_per_step = _graph_node_count(g)
-        g.instantiate()
-        self.graph = g
-        return g
+        saved, now = list(self._host_pos), self._absorbs()
+        graphs = {}
+        for absorb in ((now, not now) if self.absorb_below else (now,)):
+            if absorb != now:
+                self._host_pos = [0 if absorb else self.absorb_below]
+            g = graphs[absorb] = torch.cuda.CUDAGraph(keep_graph=True)
+            with torch.cuda.graph(g):
+                self.step()
+            self._host_pos = list(saved)
+        self.kernels_per_step = _graph_node_count(graphs[now])
+        for g in graphs.values():
+            g.instantiate()
+        self.graph, self._graphs = graphs[now], graphs
+        return self.graph
 
     def check_errors(self) -> None:
         """Raise if a kernel of the steps so far skipped a cache write past a row's capacity
@@ -812,5 +832,5 @@ class DecodeEngine:
         if self.graph is None:
             raise RuntimeError("capture() first")
         self._check_room()
-        self.graph.replay()
+        self._graphs[self._absorbs()].replay()
         self._host_pos = [p + 1 for p in self._host_pos]

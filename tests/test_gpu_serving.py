@@ -200,3 +200,43 @@ def test_small_family_absorb_and_split_decode_agree_at_the_threshold(weights):
         eng.check_errors()
         got.append(eng.logits.float().clone())
     assert float((got[0] - got[1]).abs().max() / got[0].abs().max()) < 2e-2
+
+
+def test_one_row_takes_the_path_of_its_length(weights, monkeypatch):
+    """A lone row in a cache with room to grow runs the absorb step while few tokens are cached and
+    the split-KV one from ABSORB_ROW_CTX, eagerly and replayed alike (bitwise), over the crossing and
+    after a short prompt takes the slot again."""
+    import dsv2lite
+    import dsv2lite.engine as E
+
+    calls, call = [], E.call
+    monkeypatch.setattr(E, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    start = E.ABSORB_ROW_CTX - 3
+    eng = dsv2lite.DecodeEngine(weights, [1000], family="small")
+    eng.prefill(_prompts([start], 13))
+    snap = eng.snapshot()
+    eager = []
+    for i in range(6):
+        calls.clear()
+        eng.step()
+        assert ("dsv2_qkva_absorb_bf16" in calls) == (i < 3) and ("dsv2_mla_decode" in calls) == (i >= 3), i
+        eager.append((eng.logits.clone(), eng.ids.clone()))
+    for at in (0, 4):  # captured on either side
+        eng.restore(snap)
+        for i in range(at):
+            eng.step()
+        eng.capture()
+        for i in range(at, 6):
+            calls.clear()
+            eng.replay()
+            assert not calls
+            assert torch.equal(eng.logits, eager[i][0]) and torch.equal(eng.ids, eager[i][1]), (at, i)
+    eng.insert(0, _prompts([9], 14)[0])
+    snap = eng.snapshot()
+    eng.replay()
+    got = eng.logits.clone()
+    eng.restore(snap)
+    calls.clear()
+    eng.step()
+    assert "dsv2_qkva_absorb_bf16" in calls and torch.equal(got, eng.logits)
+    eng.check_errors()
