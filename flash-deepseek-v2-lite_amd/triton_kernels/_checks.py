@@ -8,7 +8,7 @@ import torch
 
 def require_cuda(name: str, *ts: torch.Tensor) -> None:
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise NotImplementedError(f"{name} requires CUDA (HIP) tensors")
 
 

@@ -114,6 +114,13 @@ def _load() -> ctypes.CDLL:
 lib = _load()
 
 
+def _stream_handle(index: int) -> int:
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _stream_handle)
+
+
 def call(name: str, *args) -> None:
     """Invoke an entry point; raise HipKernelError with the library's message on failure."""
     rc = getattr(lib, name)(*args)
@@ -123,8 +130,10 @@ def call(name: str, *args) -> None:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
-    """hipStream_t of torch's current stream (the capture stream inside torch.cuda.graph)."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream (the capture stream inside torch.cuda.graph).  By the raw
+    handle: a torch.cuda.Stream object per call costs 2 us of host time, the handle 0.1."""
+    index = device.index if device is not None else None
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -224,30 +224,31 @@ def batched_attention_decode_q1_triton(query_states: torch.Tensor, key_states: t
     if query_states.dtype != torch.bfloat16 or key_states.dtype != torch.bfloat16 or \
             value_states.dtype != torch.bfloat16:
         raise NotImplementedError("batched_attention_decode_q1_triton supports bf16 only")
-    if query_states.ndim != 4 or key_states.ndim != 4 or value_states.ndim != 4:
+    q, k, v = query_states, key_states, value_states
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
         raise ValueError("query/key/value states must be rank-4 tensors")
-    if query_states.shape[2] != 1:
+    B, H, q_len, Dq = qs
+    if q_len != 1:
         raise ValueError("batched_attention_decode_q1_triton only supports q_len=1")
     if cache_position.numel() != 1 or cache_position.dtype != torch.long:
         raise ValueError("cache_position must be CUDA int64 tensor with one element")
-    B, H, _, Dq = query_states.shape
-    Dv = value_states.shape[3]
-    L = key_states.shape[2]
-    if key_states.shape[:2] != (B, H) or value_states.shape[:3] != (B, H, L) or key_states.shape[3] != Dq:
+    L, Dv = ks[2], vs[3]
+    if ks != (B, H, L, Dq) or vs[:3] != (B, H, L):
         raise ValueError("key/value states must be [B, H, L, Dq] / [B, H, L, Dv] matching the query")
-    for t in (query_states, key_states, value_states):
-        if t.stride(3) != 1:
-            raise NotImplementedError("batched_attention_decode_q1_triton needs a contiguous last dimension")
-    out = torch.empty((B, H, 1, Dv), device=query_states.device, dtype=query_states.dtype)
+    q_st, k_st, v_st = q.stride(), k.stride(), v.stride()
+    if q_st[3] != 1 or k_st[3] != 1 or v_st[3] != 1:
+        raise NotImplementedError("batched_attention_decode_q1_triton needs a contiguous last dimension")
+    dev = q.device
+    out = torch.empty((B, H, 1, Dv), device=dev, dtype=torch.bfloat16)
     if B == 0 or L == 0:
         return out
-    q, k, v = query_states, key_states, value_states
     ns = expanded_splits(B * H, L)
-    part = torch.empty(B, H, ns, Dv + 2, dtype=torch.float32, device=q.device) if ns > 1 else None
-    _hip.call("dsv2_attention_decode_expanded_split", q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0),
-              k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(),
-              out.stride(0), out.stride(1), B, H, Dq, Dv, L, cache_position.data_ptr(), float(softmax_scale), ns,
-              _hip.ptr(part), _expanded_status(q.device).data_ptr(), _hip.stream_ptr(q.device))
+    part = torch.empty(B * H * ns * (Dv + 2), dtype=torch.float32, device=dev) if ns > 1 else None
+    _hip.call("dsv2_attention_decode_expanded_split", q.data_ptr(), q_st[0], q_st[1], k.data_ptr(), k_st[0], k_st[1],
+              k_st[2], v.data_ptr(), v_st[0], v_st[1], v_st[2], out.data_ptr(), H * Dv, Dv, B, H, Dq, Dv, L,
+              cache_position.data_ptr(), float(softmax_scale), ns, None if part is None else part.data_ptr(),
+              _expanded_status(dev).data_ptr(), _hip.stream_ptr(dev))
     return out
 
 
@@ -257,20 +258,23 @@ def expanded_splits(pairs: int, length: int) -> int:
     buffer.  Measured on MI355X (whole calls, one range against the best of 2..16; pairs x cached
     tokens): 16 x 4000 49.2 -> 20.9 us with 8, 32 x 3000 40.7 -> 21.3 with 8, 64 x 3900 53.2 ->
     33.0 with 4; but 16 x 900 16.3 -> 20.3, 64 x 800 15.4 -> 19.6, 128 x 2000 33.3 -> 32.4 and
-    192 x 1380 29.2 -> 35.9."""
+    192 x 1380 29.2 -> 35.9.  The position is known on the device only, so a short one in a long cache
+    pays for the second launch too: 60 tokens 3.8 us with one range, 6.1 with several, and 4 us of
+    host time, which the wrapper keeps within what one launch cost it by asking torch for less."""
     if pairs > 96 or length < 1536:
         return 1
-    return max(1, min(8, length // 512, 256 // max(pairs, 1)))
+    return min(8, length // 512, 256 // max(pairs, 1))
 
 
 _EXPANDED_STATUS: dict = {}
 
 
 def _expanded_status(dev: torch.device) -> torch.Tensor:
-    k = dev.index if dev.index is not None else 0
-    if k not in _EXPANDED_STATUS:
-        _EXPANDED_STATUS[k] = torch.zeros(1, dtype=torch.int32, device=dev)
-    return _EXPANDED_STATUS[k]
+    k = dev.index or 0
+    st = _EXPANDED_STATUS.get(k)
+    if st is None:
+        st = _EXPANDED_STATUS[k] = torch.zeros(1, dtype=torch.int32, device=dev)
+    return st
 
 
 def check_expanded_status(device: torch.device | str = "cuda") -> None:

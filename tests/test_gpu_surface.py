@@ -535,3 +535,23 @@ def test_mla_kernels_never_touch_another_rows_slots():
     # row 1 (within capacity) agrees between the paths; row 0 attended its 40 rows only
     assert rel_err(c(outs["fused"][1]), c(outs["split"][1])) < 2e-2
     assert rel_err(c(outs["absorb"][1]), c(outs["split"][1])) < 2e-2
+
+
+def test_stream_ptr_is_the_current_stream():
+    """The raw handle the wrappers launch on: torch's current stream of the device -- the default one,
+    a side stream, a device without an index, the stream of a capture -- by the same value as the
+    Stream object gives."""
+    from triton_kernels import _hip
+
+    devs = (None, torch.device("cuda"), torch.device("cuda", torch.cuda.current_device()))
+    for d in devs:
+        assert _hip.stream_ptr(d) == torch.cuda.current_stream(d).cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert all(_hip.stream_ptr(d) == side.cuda_stream for d in devs)
+    seen = []
+    x = torch.zeros(4, device=DEV)
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        seen = [_hip.stream_ptr(d) == torch.cuda.current_stream(d).cuda_stream for d in devs]
+        x.add_(1)
+    assert all(seen) and _hip.stream_ptr() == torch.cuda.current_stream().cuda_stream
