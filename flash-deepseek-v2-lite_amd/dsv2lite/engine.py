@@ -363,9 +363,6 @@ class DecodeEngine:
         # one row in a longer cache: absorb below this position, split-KV from it (0: not so)
         self.absorb_below = ABSORB_ROW_CTX if (self.step_family == "small" and mla_path == "absorb" and self.B == 1 and
                                                ABSORB_MAX_CTX < self.max_pos <= FUSED_MLA_MAX_CTX) else 0
-        # the path asked for, where the cache is short enough for the one- and two-launch paths at
-        # all; "absorb" leaves caches past ABSORB_MAX_CTX to the split-KV decode as well
-        self.mla_path = mla_path if family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX else "split"
         self.max_prefill_rows = max_prefill_rows
         self.graph = None
         self._graphs: dict[bool, torch.cuda.CUDAGraph] = {}  # captured step by _absorbs()
@@ -610,6 +607,13 @@ class DecodeEngine:
             call("dsv2_gemm_bf16", ptr(b.xn), c.hidden, 0, B, c.hidden, ptr(self.w.lm_head), 0, c.vocab, 1, None, 0,
                  ptr(self.logits), c.vocab, 0, LINEAR_OUT_F32, st)
         call("dsv2_argmax_f32", ptr(self.logits), B, c.vocab, ptr(self.ids), ptr(pos), st)
+
+    @property
+    def mla_path(self) -> str:
+        """The attention path the next step runs: "split" for the batch kernels and past the caches
+        or rows the path asked for takes, else "fused", "spread" or "absorb"."""
+        return ("fused" if self.fused_mla else "spread" if self.spread_mla else
+                "absorb" if self._absorbs() else "split")
 
     def _absorbs(self) -> bool:
         """Whether the next step's attention runs the absorb path."""

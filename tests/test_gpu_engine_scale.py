@@ -60,12 +60,12 @@ def _graph_equals_eager(eng, snap, steps=2):
     eng.restore(snap)
 
 
-def _parity(model, family, lens, seed, steps=3, rows=None, graph=True, tile=None, chunk=8192):
+def _parity(model, family, lens, seed, steps=3, rows=None, graph=True, tile=None, chunk=8192, mla="absorb"):
     import dsv2lite
 
     cfg, w, om = model
     B = len(lens)
-    eng = dsv2lite.DecodeEngine(w, [n + steps + 8 for n in lens], family=family, max_prefill_rows=chunk)
+    eng = dsv2lite.DecodeEngine(w, [n + steps + 8 for n in lens], family=family, max_prefill_rows=chunk, mla_path=mla)
     P = prompts(lens, seed)
     prec = []
     first = eng.prefill([p.cuda() for p in P], record=prec).cpu().clone()
@@ -199,15 +199,32 @@ def test_replicated_prompt_rows_stay_bitwise_identical(model, B):
     eng.check_errors()
 
 
-@pytest.mark.parametrize("bsz", [8, 64])
-def test_small_family_at_larger_batches(model, bsz):
-    """The small (GEMV) family above bsz=3, as the reference runs it up to bsz=256
-    (attention_decode_small.py:932-1070, moe_small_gemv.py:430-514): ragged prompts, the
-    absorbed q|kv_a projection, the one-launch attention and the route-local MoE with 8 and
-    64 rows (the lm_head GEMV + argmax above 8 rows).  Two sampled rows (the shortest and the
-    longest prompt) against the oracle, teacher-forced for 3 steps; graph == eager for the
-    whole batch."""
+@pytest.mark.parametrize("bsz,mla,step_family,runs", [
+    (8, "absorb", "batch", "split"), (64, "absorb", "batch", "split"),  # the default: batch kernels from 5 rows
+    (8, "split", "small", "split"), (64, "split", "small", "split"),
+    (8, "fused", "small", "fused"), (64, "spread", "small", "spread")])
+def test_small_family_at_larger_batches(model, bsz, mla, step_family, runs):
+    """The small family above bsz=3, as the reference runs it up to bsz=256
+    (attention_decode_small.py:932-1070, moe_small_gemv.py:430-514), with ragged prompts: on the batch
+    family's kernels by default, and on its own -- GEMV projections, the split, fused or spread
+    attention, the route-local MoE and the lm_head GEMV + argmax with 8 and 64 rows -- where an MLA
+    path is asked for.  Two sampled rows (the shortest and the longest prompt) against the oracle,
+    teacher-forced for 3 steps; graph == eager for the whole batch."""
     g = torch.Generator().manual_seed(20 + bsz)
     lens = torch.randint(24, 600, (bsz,), generator=g).tolist()
-    eng = _parity(model, "small", lens, seed=20 + bsz, rows=_sample(lens, 20 + bsz)[:2])
-    assert eng.mla_path == "absorb"
+    eng = _parity(model, "small", lens, seed=20 + bsz, rows=_sample(lens, 20 + bsz)[:2], mla=mla)
+    assert eng.step_family == step_family and eng.mla_path == runs
+
+
+@pytest.mark.parametrize("rows,cap,mla,runs", [
+    (1, 600, "absorb", "absorb"), (4, 640, "absorb", "absorb"), (4, 641, "absorb", "split"), (1, 700, "absorb", "absorb"),
+    (1, 2049, "absorb", "split"), (2, 2048, "fused", "fused"), (2, 2049, "fused", "split"), (5, 64, "absorb", "split"),
+    (5, 64, "spread", "spread")])
+def test_mla_path_names_the_path_that_runs(model, rows, cap, mla, runs):
+    import dsv2lite
+
+    eng = dsv2lite.DecodeEngine(model[1], [cap] * rows, family="small", mla_path=mla)
+    assert eng.mla_path == runs
+    if (rows, cap) == (1, 700):  # a lone row's path follows its length
+        eng._host_pos = [384]
+        assert eng.mla_path == "split"
