@@ -14,8 +14,8 @@ token prompts, batch family) -- timed in the same run on the same weights, each 
 tok/s, ms/step, step roofline and dominant-kernel roofline.  --config N runs one config
 alone; r64|r256 are the reference's own published workload (one 24-token prompt replicated
 over the batch), whose vs_baseline is value / the published A100 batch-family TPS for it,
-and s8|s64 the same workload on the small (GEMV) family, against the published A100
-small-GEMV TPS.  The default line carries all of them under "configs", with the isolated
+and s8|s64 the same workload on the small family (from 5 rows its step runs the batch
+kernels), against the published A100 small-GEMV TPS.  The default line carries all of them under "configs", with the isolated
 MLA microbenchmark (C4) and configs 1-3 again on e4m3 expert weights (C1_fp8..C3_fp8).
 --config 4 is the isolated absorbed-MLA decode microbenchmark (bsz=128, KV lengths
 U[256,8192]); its value is compressed-cache GB/s.
@@ -71,7 +71,8 @@ CONFIGS = {
     "r256": dict(batch=256, family="batch", prompt=lambda g: [24] * 256, seed=4, replicate=True, published=11428.26,
                  workload="reference workload: bsz=256, one 24-token random prompt replicated, batch family, "
                           "hipGraph"),
-    # the same workload on the small (GEMV) family above bsz=1; published: the A100 "forced
+    # the same workload on the small family above bsz=1 (its step runs the batch kernels from 5
+    # rows; --mla-path split|fused|spread keeps its GEMV kernels); published: the A100 "forced
     # small-GEMV" column of docs/third_party_baselines.md:90-100
     "s8": dict(batch=8, family="small", prompt=lambda g: [24] * 8, seed=4, replicate=True, published=614.82,
                workload="reference workload: bsz=8, one 24-token random prompt replicated, small family, hipGraph"),
@@ -292,7 +293,7 @@ def time_other_kernels(eng, family: str, ctx_rows: list[int]) -> dict:
     entry("expert-grouped down" + (" on e4m3 weights" if fp8 else "") + (" + the 2 shared-expert halves" if shared else "")
           + f" ({b.tile_tokens}-token tiles)", down, moe, nb)
 
-    if b.max_splits == 1:
+    if b.max_splits == 1 and eng.family == "batch":  # the small family merges into fp32 o_lat and W_UV
         def decode(li):
             call("dsv2_mla_decode_rows", ptr(b.q), ptr(eng.cache.layer(li)), ptr(eng.cache.base), ptr(eng.cache.pos),
                  ptr(eng.cache.cap), B, eng.scale, ptr(b.olat), 16 * 512, stream_ptr())
@@ -799,7 +800,7 @@ def run_config(key, w, args, cfg, dev, expert_dtype: str = "bf16") -> dict:
     others = time_other_kernels(eng, eng.step_family, [p + 1 for p in pos_now])
     res = {"workload": spec["workload"] + (", e4m3 expert weights" if expert_dtype == "fp8" else ""),
            "expert_dtype": expert_dtype, "global_batch": B, "seq_len": max(lens), "kernel_family": family,
-           "mla_path": args.mla_path if eng.step_family == "small" else "split", "prompt_tokens": sum(lens),
+           "mla_path": eng.mla_path, "prompt_tokens": sum(lens),
            "tok_s": value, "ms_per_step": ms, "steps": steps, "warmup": warm, "kernels_per_step": eng.kernels_per_step,
            "roofline": roof,
            "other_kernels": others,

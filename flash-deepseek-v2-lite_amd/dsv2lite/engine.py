@@ -123,19 +123,9 @@ class PrefillPlan:
         self.kexp, self.vexp = kexp, vexp
 
 
-def _segments(seq: torch.Tensor, posv: torch.Tensor) -> list[tuple[int, int, int, int]]:
-    """(first chunk row, rows, sequence, first position) of each run of one sequence's rows in a
-    chunk."""
-    vals, counts = torch.unique_consecutive(seq, return_counts=True)
-    out, r = [], 0
-    for s, cnt in zip(vals.tolist(), counts.tolist()):
-        out.append((r, cnt, s, int(posv[r])))
-        r += cnt
-    return out
-
-
 def _chunk_segments(lens: list[int], s: int, e: int) -> list[tuple[int, int, int, int]]:
-    """_segments of rows [s, e) of prompts of the given lengths laid one after the other."""
+    """(first chunk row, rows, sequence, first position) of each sequence's rows in the chunk of rows
+    [s, e) of prompts of the given lengths laid one after the other."""
     out, start = [], 0
     for j, n in enumerate(lens):
         lo, hi = max(s, start), min(e, start + n)
@@ -145,7 +135,10 @@ def _chunk_segments(lens: list[int], s: int, e: int) -> list[tuple[int, int, int
     return out
 
 
-def _group_tiles(segs, bases: list[int], tile: int) -> tuple[list[tuple[int, int, int, int]], int, int]:
+def _group_tiles(segs, bases: list[int], tile: int = 128) -> tuple[list[tuple[int, int, int, int]], int, int]:
+    """Query tiles of a chunk's segments (first chunk row, rows, first position, cache base) and the
+    cache row range [lo, lo + n) their attention reads: from the lowest sequence base to the last
+    position of any row."""
     out, lo, hi = [], None, None
     for r, cnt, s, p_first in segs:
         for a in range(0, cnt, tile):
@@ -159,6 +152,10 @@ def _group_tiles(segs, bases: list[int], tile: int) -> tuple[list[tuple[int, int
 
 def _plan_groups(segs, bases: list[int], tile: int = 128,
                  slack: int = 4096) -> list[tuple[list[tuple[int, int, int, int]], int, int]]:
+    """_group_tiles in groups of consecutive sequences whose expanded cache range stays within
+    twice the rows they attend (plus `slack`): with slots far apart (capacities much larger
+    than the prompts) one range over the whole chunk would expand every slot's unused
+    capacity in between.  Each group: (tiles, exp_lo, exp_rows)."""
     groups, cur, lo, hi, used = [], [], 0, 0, 0
     for seg in segs:
         _, cnt, s, p_first = seg
@@ -177,23 +174,6 @@ def _plan_groups(segs, bases: list[int], tile: int = 128,
 
 def _tile_tensor(tiles: list[tuple[int, int, int, int]]) -> torch.Tensor:
     return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 4)
-
-
-def prefill_tiles(seq: torch.Tensor, posv: torch.Tensor, bases: list[int], tile: int = 128) -> tuple[torch.Tensor, int, int]:
-    """Query tiles of one chunk (seq[r]: sequence of chunk row r, posv[r]: its position;
-    rows of a sequence are consecutive with consecutive positions) and the cache row range
-    its attention reads: from the lowest sequence base to the last position of any row."""
-    t, lo, n = _group_tiles(_segments(seq, posv), bases, tile)
-    return _tile_tensor(t), lo, n
-
-
-def prefill_groups(seq: torch.Tensor, posv: torch.Tensor, bases: list[int], tile: int = 128,
-                   slack: int = 4096) -> list[tuple[torch.Tensor, int, int]]:
-    """prefill_tiles in groups of consecutive sequences whose expanded cache range stays within
-    twice the rows they attend (plus `slack`): with slots far apart (capacities much larger
-    than the prompts) one range over the whole chunk would expand every slot's unused
-    capacity in between.  Each group: (tiles, exp_lo, exp_rows)."""
-    return [(_tile_tensor(t), lo, n) for t, lo, n in _plan_groups(_segments(seq, posv), bases, tile, slack)]
 
 
 class _Upload:

@@ -351,7 +351,7 @@ def test_prefill_tiles_cover_every_row_once():
     """The prefill attention's query tiles: <= 128 consecutive rows of one sequence each, every
     chunk row in exactly one tile with its own position and its sequence's cache base; the
     expanded range spans every key any row attends."""
-    from dsv2lite.engine import prefill_tiles
+    from dsv2lite.engine import _chunk_segments, _group_tiles
 
     lens = [100, 3, 64, 130]
     bases = [0, 200, 300, 500]
@@ -359,9 +359,9 @@ def test_prefill_tiles_cover_every_row_once():
     posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
     # a chunk that starts inside sequence 0 (positions 40..) and ends inside sequence 3
     s, e = 40, 100 + 3 + 64 + 70
-    t, lo, n = prefill_tiles(seq[s:e], posv[s:e], bases)
+    t, lo, n = _group_tiles(_chunk_segments(lens, s, e), bases)
     seen = torch.zeros(e - s, dtype=torch.int32)
-    for r0, nr, p0, sb in t.tolist():
+    for r0, nr, p0, sb in t:
         assert 1 <= nr <= 128
         rows = torch.arange(r0, r0 + nr)
         assert len(set(seq[s:e][rows].tolist())) == 1
@@ -378,7 +378,7 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
     groups whose expanded cache range is at most twice the rows they attend plus the slack,
     instead of one range over every slot's unused capacity (64 x 32768 rows); the groups
     together cover every chunk row exactly once.  Slots packed closely stay one group."""
-    from dsv2lite.engine import prefill_groups, prefill_tiles
+    from dsv2lite.engine import _chunk_segments, _group_tiles, _plan_groups
 
     def plan(lens, caps, slack=4096):
         bases = [0]
@@ -386,7 +386,7 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
             bases.append(bases[-1] + c)
         seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(lens)])
         posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
-        return seq, posv, bases, prefill_groups(seq, posv, bases, slack=slack)
+        return seq, posv, bases, _plan_groups(_chunk_segments(lens, 0, sum(lens)), bases, slack=slack)
 
     lens = [100] * 64
     seq, posv, bases, groups = plan(lens, [32768] * 64)
@@ -394,7 +394,7 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
     total_exp = 0
     for tiles, lo, n in groups:
         used = 0
-        for r0, nr, p0, sb in tiles.tolist():
+        for r0, nr, p0, sb in tiles:
             seen[r0:r0 + nr] += 1
             assert lo <= sb and sb + p0 + nr <= lo + n  # every key of the tile's rows is expanded
             used += nr
@@ -402,24 +402,30 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
         total_exp += n
     assert torch.all(seen == 1)
     assert total_exp <= 64 * 100 + 64 * 4096 and total_exp < 64 * 32768 // 4
-    # bench-like capacities (prompt + a few tokens): one group, the same plan as prefill_tiles
+    # bench-like capacities (prompt + a few tokens): one group, the plan of all the rows together
     seq, posv, bases, groups = plan([2048] * 4, [2081] * 4)
-    assert len(groups) == 1
-    t, lo, n = prefill_tiles(seq, posv, bases)
-    assert torch.equal(groups[0][0], t) and groups[0][1:] == (lo, n)
+    assert groups == [_group_tiles(_chunk_segments([2048] * 4, 0, 4 * 2048), bases)]
 
 
 def test_chunk_segments_equal_the_rows_own_runs():
     """The chunk plan from prompt lengths alone equals the one read off the chunk's per-row
     sequence and position tensors, for every cut of ragged prompts."""
-    from dsv2lite.engine import _chunk_segments, _segments
+    from dsv2lite.engine import _chunk_segments
+
+    def runs(seq, posv):
+        vals, counts = torch.unique_consecutive(seq, return_counts=True)
+        out, r = [], 0
+        for v, cnt in zip(vals.tolist(), counts.tolist()):
+            out.append((r, cnt, v, int(posv[r])))
+            r += cnt
+        return out
 
     lens = [5, 1, 17, 9]
     seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(lens)])
     posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])
     for s in range(sum(lens)):
         for e in range(s + 1, sum(lens) + 1):
-            assert _chunk_segments(lens, s, e) == _segments(seq[s:e], posv[s:e])
+            assert _chunk_segments(lens, s, e) == runs(seq[s:e], posv[s:e])
 
 
 def _mfma_hazards():

@@ -1096,7 +1096,7 @@ def test_mla_prefill_attention_vs_fp32(lens, start):
     """Prefill attention (expanded form, causal) against fp32 torch: rows of several
     sequences (a chunk that may start inside the first sequence: its earlier keys come from
     the cache), 128-query tiles with partial last tiles."""
-    from dsv2lite.engine import prefill_tiles
+    from dsv2lite.engine import _chunk_segments, _group_tiles, _tile_tensor
 
     caps = [n + 30 for n in lens]
     bases = [0]
@@ -1106,7 +1106,7 @@ def test_mla_prefill_attention_vs_fp32(lens, start):
     seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(lens)])[start:]
     posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens])[start:]
     R = seq.numel()
-    tiles, lo, nexp = prefill_tiles(seq, posv, bases)
+    tiles, lo, nexp = _group_tiles(_chunk_segments(lens, start, sum(lens)), bases)
     cache = rnd(ncache, 576, seed=200)
     kexp = rnd(nexp, 16, 128, seed=201)
     vexp = rnd(nexp, 16, 128, seed=202)
@@ -1114,7 +1114,7 @@ def test_mla_prefill_attention_vs_fp32(lens, start):
     qrope = rnd(R, 16, 576, seed=204)
     out = torch.full((R, 2048), float("nan"), dtype=BF, device=DEV)
     scale = O.softmax_scale(O.Dims())
-    td = tiles.to(DEV)
+    td = _tile_tensor(tiles).to(DEV)
     call("dsv2_mla_prefill_attention", qkva.data_ptr(), 3648, qrope.data_ptr(), 16 * 576, R, cache.data_ptr(), ncache,
          kexp.data_ptr(), vexp.data_ptr(), lo, nexp, td.data_ptr(), td.shape[0], scale, out.data_ptr(), 2048, st())
     c = lambda t: t.float().cpu()  # noqa: E731
@@ -1144,18 +1144,24 @@ def test_stream_copy_exact(nbytes):
     assert torch.all(dst[nbytes:] == 7)
 
 
-@pytest.mark.parametrize("rows,K,N,swiglu,out", [
-    (2300, 704, 3648, False, "bf16"),      # odd K chunks, a ragged last feature block, 192-token tiles
-    (2300, 704, 3648, False, "residual"),
-    (2300, 704, 3648, False, "narrow"),    # 8-byte aligned output and residual rows
-    (4100, 192, 2080, True, "bf16"),       # SwiGLU, the last block a quarter full, 3 K chunks
-    (8129, 64, 4096, False, "f32"),        # one K chunk, several items per workgroup
-    (5000, 128, 2048, False, "exact"),
+@pytest.mark.parametrize("rows,K,N,swiglu,out,tiles", [
+    (2300, 704, 3648, False, "bf16", 3),      # 11 K chunks, a ragged last feature block
+    (2300, 704, 3648, False, "residual", 3),
+    (2300, 704, 3648, False, "narrow", 3),    # 8-byte aligned output and residual rows
+    (4100, 192, 2080, True, "bf16", 3),       # SwiGLU, the last block a quarter full, 3 K chunks
+    (8129, 128, 8256, False, "f32", 4),       # 2 and 12 chunks: several items per workgroup, each prefetching
+    (8129, 128, 8256, False, "bf16", 4),      # the next one's first two chunks; the last block a quarter full
+    (5001, 768, 8256, False, "exact", 4),
+    (5001, 768, 4160, True, "bf16", 4),
 ])
-def test_large_tile_gemm_edges(rows, K, N, swiglu, out):
-    """Shapes whose cost picks the 256-row tiles, against fp32 torch: one bf16 round of an fp32 sum
-    is 2^-9 of the value (4e-3 of the largest bounds it), with a residual there are two (the sum,
-    then sum + residual: 8e-3), with SwiGLU four (1e-2)."""
+def test_large_tile_gemm_edges(rows, K, N, swiglu, out, tiles):
+    """Shapes whose cost picks the 256-row tiles (`tiles` x 64 tokens each), against fp32 torch: one
+    bf16 round of an fp32 sum is 2^-9 of the value (4e-3 of the largest bounds it), with a residual
+    there are two (the sum, then sum + residual: 8e-3), with SwiGLU four (1e-2)."""
+    assert _hip.lib.dsv2_gemm_dense_tiles(rows, K, N, 1 if swiglu else 0) == tiles
+    rows_wg = 128 if swiglu else 256
+    items = -(-rows // (64 * tiles)) * -(-N // rows_wg)
+    assert K // 64 % 2 or items > 256  # an even number of chunks: a persistent grid of several rounds
     x, w = rnd(rows, K, seed=90), rnd((2 if swiglu else 1) * N, K, seed=91, std=K ** -0.5)
     ld = N + 4 if out == "narrow" else N
     flags = {"f32": 2, "exact": 4}.get(out, 0) | (1 if swiglu else 0)
@@ -1171,7 +1177,25 @@ def test_large_tile_gemm_edges(rows, K, N, swiglu, out):
     assert rel_err(y[:, :N].float(), ref) < {"exact": 1e-5}.get(out, 1e-2 if swiglu else (8e-3 if res is not None else 4e-3))
 
 
-@pytest.mark.parametrize("inter", [128, 192])
+@pytest.mark.parametrize("K,N", [(2048, 3648), (704, 3648)])
+def test_dense_tile_shapes_sum_k_in_the_same_order(K, N):
+    """The 64 x 64 ring (but for weights of tens of MB, whose K chunks it rotates) and the large tiles
+    of every token count add each output's products in K order: a row's result is the same bits
+    whichever of them its launch takes, with odd and even numbers of K chunks."""
+    rows = {}
+    for r in range(128, 16385, 64):
+        rows.setdefault(_hip.lib.dsv2_gemm_dense_tiles(r, K, N, 0), r)
+    assert {0, 4} <= set(rows) and len(rows) >= 4, rows
+    x, w = rnd(max(rows.values()), K, seed=96), rnd(N, K, seed=97, std=K ** -0.5)
+    got = []
+    for r in rows.values():
+        y = torch.empty(r, N, device=DEV)
+        call("dsv2_gemm_bf16", x.data_ptr(), K, 0, r, K, w.data_ptr(), 0, N, 1, None, 0, y.data_ptr(), N, 0, 4, st())
+        got.append(y[:min(rows.values())])
+    assert all(torch.equal(got[0], y) for y in got[1:]), rows
+
+
+@pytest.mark.parametrize("inter", [64, 128, 192])
 def test_grouped_large_tile_token_counts(inter):
     """256-token expert tiles holding 1 to 256 tokens (each of the kernel's token loops and its
     edges) against the same routes on 64-token tiles: the gate_up and down products are the same
@@ -1198,7 +1222,7 @@ def test_grouped_large_tile_token_counts(inter):
             call("dsv2_moe_grouped_gateup", x.data_ptr(), srt.data_ptr(), tiles.data_ptr(), nt.data_ptr(), n, tile,
                  gu.data_ptr(), inter, hs.data_ptr(), st())
         else:
-            hs = got[64][0]  # 256-token gate_up tiles need inter % 128: only the down (odd K chunks)
+            hs = got[64][0]  # 256-token gate_up tiles need inter % 128: only the down (1 and 3 K chunks)
         call("dsv2_moe_grouped_down", (got[64][0] if tile == 256 else hs).data_ptr(), tiles.data_ptr(), nt.data_ptr(), n,
              tile, dn.data_ptr(), inter, ys.data_ptr(), st())
         got[tile] = (hs, ys)
@@ -1212,7 +1236,7 @@ def test_mla_prefill_query_tile_sizes_agree_bitwise(lens):
     """Few query tiles run as halves of 64 queries, 32 and more as whole tiles: the same sequences
     alone and beside enough one-token sequences for whole tiles give the same bits, and both are
     within 1e-2 of fp32 attention (bf16 probabilities and output, 2^-9 each)."""
-    from dsv2lite.engine import prefill_tiles
+    from dsv2lite.engine import _chunk_segments, _group_tiles, _tile_tensor
 
     outs = []
     for extra in (0, 33):
@@ -1221,15 +1245,13 @@ def test_mla_prefill_query_tile_sizes_agree_bitwise(lens):
         for n in ls[:-1]:
             bases.append(bases[-1] + n)
         R, total = sum(ls), sum(ls)
-        seq = torch.cat([torch.full((n,), b, dtype=torch.int64) for b, n in enumerate(ls)])
-        posv = torch.cat([torch.arange(n, dtype=torch.int32) for n in ls])
-        tiles, lo, nexp = prefill_tiles(seq, posv, bases)
-        assert (tiles.shape[0] >= 32) == (extra > 0)
+        tiles, lo, nexp = _group_tiles(_chunk_segments(ls, 0, R), bases)
+        assert (len(tiles) >= 32) == (extra > 0)
         full = total if extra else total + 33  # the same leading rows in both
         cache, ke, ve = rnd(full, 576, seed=210), rnd(full, 16, 128, seed=211), rnd(full, 16, 128, seed=212)
         qkva, qrope = rnd(full, 3648, seed=213), rnd(full, 16, 576, seed=214)
         out = torch.full((full, 2048), float("nan"), dtype=BF, device=DEV)
-        td = tiles.to(DEV)
+        td = _tile_tensor(tiles).to(DEV)
         call("dsv2_mla_prefill_attention", qkva.data_ptr(), 3648, qrope.data_ptr(), 16 * 576, R, cache.data_ptr(), full,
              ke.data_ptr(), ve.data_ptr(), lo, nexp, td.data_ptr(), td.shape[0], 0.1147, out.data_ptr(), 2048, st())
         outs.append(out[:sum(lens)].clone())
@@ -1291,6 +1313,24 @@ def test_mla_decode_equal_pieces(split, lens):
     call("dsv2_mla_decode_rows", P(q), P(cache), P(base), P(pos), P(capd), B, 0.1147, P(outs[1]), 8192, st())
     assert torch.isfinite(outs[0].float()).all()
     assert rel_err(outs[0].float(), outs[1].float()) < 2 ** -7
+
+
+def test_bf16_rounding_equals_torch_for_every_fp32_value():
+    """The kernels' fp32 -> bf16 conversion over all 2^32 bit patterns, through the split merge of one
+    split (its weight is exactly 1): torch's round-to-nearest-even value, NaN for NaN, subnormals and
+    infinities included."""
+    rows, n = 32768, 32768 * 8192  # 2^28 values a call
+    ml = torch.tensor([0.0, 1.0], device=DEV).repeat(rows * 16)
+    pos, cap = torch.zeros(rows, dtype=torch.int32, device=DEV), torch.ones(rows, dtype=torch.int32, device=DEV)
+    out = torch.empty(n, dtype=BF, device=DEV)
+    for part in range(16):
+        bits = torch.arange(n, dtype=torch.int32, device=DEV) + (part * n - 2 ** 31)
+        x = bits.view(torch.float32)
+        call("dsv2_mla_combine", x.data_ptr(), ml.data_ptr(), pos.data_ptr(), cap.data_ptr(), rows, 32, 1, None,
+             out.data_ptr(), 8192, st())
+        want = x.to(BF)
+        assert torch.equal(torch.isnan(out), torch.isnan(want)), part
+        assert torch.all((out == want) | torch.isnan(want)), part
 
 
 @pytest.mark.parametrize("rows,splits", [(30, 16), (31, 16), (120, 4), (121, 4), (240, 2), (241, 2)])
