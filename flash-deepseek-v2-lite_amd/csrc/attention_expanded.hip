@@ -13,7 +13,8 @@
 // done, then the 8 groups of a wave meet by lane swaps and the 8 waves in LDS; fp32
 // throughout, one bf16 round.  (Staging 64-token chunks through LDS with three barriers each kept
 // one chunk's loads in flight at a time.)  MI355X, 12 rows x 16 heads x 1,381 tokens of 192 + 128
-// dims (170 MB): 178 -> 35 us, 4.9 TB/s.
+// dims (170 MB): 178 -> 28 us with five such caches read in turn (6.0 TB/s; the same one again 26,
+// partly from the last-level cache).
 #include "common.h"
 
 namespace {

@@ -422,8 +422,8 @@ __device__ __forceinline__ void gemm_store4(const GemmArgs& a, int g, int slot, 
   gemm_store4r(a, g, slot, n, v, a.res ? *reinterpret_cast<const uint2*>(a.res + (int64_t)slot * a.rs + n) : uint2{0u, 0u});
 }
 
-// Direct-to-LDS ring shape for dense weights at 128+ tokens (the lm_head from 33) and for the
-// expert-grouped MoE's 64-token tiles: a 4-wave workgroup owns 64
+// Direct-to-LDS ring shape for dense weights from 65 tokens (the lm_head and the dense gate_up from
+// 33; dense_tiles) and for the expert-grouped MoE's 64-token tiles: a 4-wave workgroup owns 64
 // features x 64 tokens (each wave 32 x 32, 2 x 2 MFMA blocks).  K streams in 64-wide chunks
 // through a ring of kDmaStages 16 KB LDS stages filled by global_load_lds (16 bytes per
 // lane straight into LDS, no register round trip): every load covers 8 rows x 128 B, and

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
   const int nkv = p0 + nr;  // keys [0, nkv) of the sequence
   const int ntiles = (nkv + kKT - 1) / kKT;
 
-  // K/V tiles stream straight into a 3-stage LDS ring (global_load_lds, 16 B per lane): ring
+  // K/V tiles stream straight into a 4-stage LDS ring (global_load_lds, 16 B per lane): ring
   // load i of wave wv fills slots 64 (4i + wv) .. + 63 of a stage, slot s holding K chunk
   // slot s % 24 of key s / 24 (s < 768), else V chunk slot (s - 768) % 16 of key
   // (s - 768) / 16; each lane fetches the chunk that belongs in its slot
@@ -118,8 +118,8 @@ __global__ __launch_bounds__(256, 2) void mla_prefill_kernel(
                                        16, 0, 0);
     }
   };
-  // tiles past the last one repeat its keys into a stage nobody reads: every wave then has
-  // exactly kLoads newer loads in flight at each wait
+  // tiles past the last one repeat its keys (the last pass scores one such repeat and drops the
+  // result), so that every wave has exactly kLoads newer loads in flight at each wait
   issue(0, 0);
   issue(1, 1);
   issue(2, 2);

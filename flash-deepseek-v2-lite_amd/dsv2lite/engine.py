@@ -41,21 +41,23 @@ FUSED_MLA_MAX_CTX = 2048
 # small family, "absorb": caches up to this many tokens.  Its attention launch gives each of a
 # head's four workgroups every cached token; the split-KV decode spreads them over 64 splits and
 # costs two launches more.  Measured on MI355X, four-layer steps, absorb against split at 64 / 256 /
-# 560 / 1000 / 2000 cached tokens: 1 row 252 vs 268 us, 268 vs 273, 284 vs 278, 309 vs 283, 365 vs
-# 301; 4 rows 491 vs 502, 507 vs 505, 524 vs 512, 552 vs 521, 608 vs 542
+# 560 / 1000 / 2000 cached tokens: 1 row 253 vs 268 us, 269 vs 271, 285 vs 276, 309 vs 284, 361 vs
+# 296; 4 rows 494 vs 504, 510 vs 508, 527 vs 515, 553 vs 524, 609 vs 546
 ABSORB_MAX_CTX = 640
 # one row in a longer cache (up to FUSED_MLA_MAX_CTX): absorb while fewer tokens than this are
-# cached, split from there -- the step follows the row's length, not the room it has to grow (400
-# tokens 276 vs 275 us).  2 to 4 rows differ by 3% at most below the crossing and take the split path
+# cached, split from there -- the step follows the row's length, not the room it has to grow (384
+# tokens 275 vs 273 us).  2 to 4 rows differ by 3% at most below the crossing and take the split path
 # throughout, so that a row's results do not depend on the others' lengths
 ABSORB_ROW_CTX = 384
 # small family (default MLA path): from this many rows the step runs the batch family's kernels.
 # The GEMV kernels read a routed expert's weights once per row that chose it and repeat the
 # dense dot products per row on the VALU (lm_head at 8 rows 174 us against 86 on MFMA, dense
 # gate_up 65 against 19, the expert launches 160 against 121).  Measured on MI355X, four-layer
-# steps (contexts 24..600 / 300..1800), small against batch kernels: 4 rows 548 vs 591 us / 613 vs
-# 604, 5 rows 696 vs 615 / 755 vs 599, 8 rows 983 vs 707 / 1104 vs 731, 12 rows 1447 vs 769; e4m3
-# experts 4 rows 452 vs 471 / 518 vs 485, 5 rows 575 vs 494 / 643 vs 475
+# steps (contexts 24..600 / 300..1800), small against batch kernels: 4 rows 513 vs 553 us / 535 vs
+# 566, 5 rows 665 vs 590 / 676 vs 599, 8 rows 905 vs 680 / 917 vs 695, 12 rows 1311 vs 771; e4m3
+# experts 4 rows 426 vs 446 / 448 vs 466, 5 rows 558 vs 467 / 567 vs 475.  The latent output stays in
+# fp32 up to W_UV on either (merge + W_UV in one launch: 64 rows 2 to 7% of the step more than through
+# a bf16 latent and a GEMM, 16 rows none)
 SMALL_BATCH_ROWS = 5
 # batch family: up to this many rows the router runs as logits over 16 workgroups per token
 # plus a one-wave top-6 per row (64 rows: 8.3 us vs 11.1 us for one workgroup per token on
@@ -67,8 +69,9 @@ GEMM_ROUTER_MIN_ROWS = 1024
 # is VALU-bound there: 8192 rows 74 us, against three short launches)
 WIDE_BUCKET_MIN_ROWS = 1024
 # grouped MoE: from this many routes in a launch the 256-token tiles beat the 64-token ones.  The
-# crossover follows the launch's routes rather than their spread over the experts: measured on
-# MI355X with an earlier, slower form of the large-tile kernel, routed gate_up + down,
+# crossover follows the launch's routes more than their spread over the experts (a caller's own
+# routing may prefer a few: batched_grouped_routed_moe changes over later): measured on MI355X with
+# an earlier, slower form of the large-tile kernel, routed gate_up + down,
 # uniform routing (all 64 experts) 4096 routes 297 vs 321 us (64 vs 256 tokens), 6144 routes
 # 421 vs 358 us, 49152 routes 2264 vs 1155 us; every row on the same 6 experts 3072 routes
 # 109 vs 120 us, 6144 routes 213 vs 194 us

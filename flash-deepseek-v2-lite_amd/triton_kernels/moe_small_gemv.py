@@ -1,6 +1,6 @@
-"""Routed MoE, small family: route-local GEMV (reference:
-triton_kernels/moe_small_gemv.py:430-614).  Gate and up rows are paired by
-index (row i of gate with row i of up), the packing of pack_routed_experts."""
+"""Routed MoE, small family (reference: triton_kernels/moe_small_gemv.py:430-614): route-local
+GEMV up to ROUTE_GEMV_MAX_TOKENS tokens, the expert-grouped kernels above.  Gate and up rows are
+paired by index (row i of gate with row i of up), the packing of pack_routed_experts."""
 
 from __future__ import annotations
 
