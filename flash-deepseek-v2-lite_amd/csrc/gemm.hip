@@ -670,10 +670,13 @@ static void launch_dma(const GemmArgs& a, bool swiglu, hipStream_t st, int max_t
 // expert's tiles in a row), are cut into 8 contiguous ranges, one per XCD (workgroup i runs on XCD
 // i % 8): the ~32 items an XCD runs at once share each token chunk among the tile's feature blocks
 // and each weight chunk among the expert's tiles in that XCD's L2.
-// Bound: MFMA issue at the clock the power limit leaves (8192 x 10944 x 2048: 1.41 PFLOP/s at 1.88
-// GHz, MFMA busy 70%; hipBLASLt 1.57 at 1.74 GHz, 83%).  MI355X, against 8 waves of 64 x 128 (two
-// per SIMD) on one barrier and one burst of LDS reads per half chunk: 8192 x 2048 x 2048 67.5 ->
-// 63.4 us, x 2816 x 2048 88 -> 78, routed gate_up of 8,192 tokens 640 -> 600, down 385 -> 328.
+// Bound: MFMA issue in the K loop, and around it what a lone wave per SIMD cannot hide: the next
+// item's row lookups and the epilogue.  MI355X, 8192 tokens: 2048 features, K = 10944 1.39 PFLOP/s
+// (the library 1.64); 3648, K = 2048 1.19 (1.10); 10944 SwiGLU, K = 2048 1.14; counters over the last
+// products of a 256 x 2,048-token prefill: matrix cores busy 40% of its SwiGLU launches' cycles (1.16
+// PFLOP/s), 32% of the plain ones'.  Against 8 waves of 64 x 128 (two per SIMD) on one barrier and one
+// burst of LDS reads per half chunk: 8192 x 2048 x 2048 67.5 -> 55.7 us, routed gate_up of 8,192
+// tokens 640 -> 600, down 385 -> 328.
 // Four waves of 128 x 128 read 20% less LDS but cannot skip a short tile's missing tokens.
 constexpr int kBigRows = 256, kBigTokens = 256, kBigStage = (kBigRows + kBigTokens) * 128, kBigWgs = 256;
 struct BigShape {
