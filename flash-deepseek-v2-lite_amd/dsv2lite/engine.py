@@ -332,8 +332,9 @@ class DecodeEngine:
             # the small family keeps this tile whatever its rows route to, so a row's results do not
             # depend on the batch it was captured with
             self.buf.set_tile_tokens(self._fit_tile(self.buf.tile_tokens))
-        self._amax = torch.empty(max(0, _hip.lib.dsv2_lm_head_argmax_workspace_size(min(self.B, 8))),
-                                 dtype=torch.uint8, device=device)
+        # workspace of the lm_head GEMV + argmax (_head: the small family's own steps of up to 8 rows)
+        self._amax = torch.empty(_hip.lib.dsv2_lm_head_argmax_workspace_size(self.B)
+                                 if self.step_family == "small" and self.B <= 8 else 0, dtype=torch.uint8, device=device)
         # small family: one fused workgroup per (row, head) while contexts are short; the
         # split-KV kernel (parallel over the context) takes over for long contexts
         self.fused_mla = family == "small" and self.max_pos <= FUSED_MLA_MAX_CTX and mla_path == "fused"

@@ -225,6 +225,7 @@ def test_mla_path_names_the_path_that_runs(model, rows, cap, mla, runs):
 
     eng = dsv2lite.DecodeEngine(model[1], [cap] * rows, family="small", mla_path=mla)
     assert eng.mla_path == runs
+    assert (eng._amax.numel() > 0) == (eng.step_family == "small")  # rows <= 8 here
     if (rows, cap) == (1, 700):  # a lone row's path follows its length
         eng._host_pos = [384]
         assert eng.mla_path == "split"
