@@ -783,13 +783,14 @@ class DecodeEngine:
             self.tune_moe_tiles()
         saved, now = list(self._host_pos), self._absorbs()
         graphs = {}
-        for absorb in ((now, not now) if self.absorb_below else (now,)):
-            if absorb != now:
-                self._host_pos = [0 if absorb else self.absorb_below]
-            g = graphs[absorb] = torch.cuda.CUDAGraph(keep_graph=True)
-            with torch.cuda.graph(g):
-                self.step()
-            self._host_pos = list(saved)
+        try:
+            for absorb in ((now, not now) if self.absorb_below else (now,)):
+                self._host_pos = list(saved) if absorb == now else [0 if absorb else self.absorb_below]
+                g = graphs[absorb] = torch.cuda.CUDAGraph(keep_graph=True)
+                with torch.cuda.graph(g):
+                    self.step()
+        finally:  # also after a recording that failed: no row has moved
+            self._host_pos = saved
         self.kernels_per_step = _graph_node_count(graphs[now])
         for g in graphs.values():
             g.instantiate()

@@ -287,6 +287,40 @@ def test_engine_capacity_check_is_per_row():
         eng._check_room()
 
 
+def test_failed_capture_leaves_positions_and_graphs(monkeypatch):
+    """capture() records the form of the other side of ABSORB_ROW_CTX at a position of its own; a
+    recording that fails leaves the row where it is and the earlier graphs in place."""
+    import contextlib
+    from types import SimpleNamespace
+
+    from dsv2lite.engine import DecodeEngine
+
+    eng = object.__new__(DecodeEngine)
+    eng.family, eng.absorb_mla, eng.absorb_below, eng._host_pos = "small", False, 384, [17]
+    eng.graph, eng._graphs = None, {}
+    seen = []
+
+    def step():
+        seen.append(eng._host_pos[0])
+        if len(seen) == fails_at:
+            raise RuntimeError("recording failed")
+        eng._host_pos = [eng._host_pos[0] + 1]
+
+    eng.step = step
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda keep_graph: SimpleNamespace(instantiate=lambda: None))
+    monkeypatch.setattr(torch.cuda, "graph", lambda g: contextlib.nullcontext())
+    monkeypatch.setattr("dsv2lite.engine._graph_node_count", lambda g: 1)
+    for fails_at in (1, 2):
+        seen.clear()
+        with pytest.raises(RuntimeError, match="recording failed"):
+            eng.capture()
+        assert eng._host_pos == [17] and eng.graph is None and eng._graphs == {}
+    fails_at = 0
+    seen.clear()
+    assert eng.capture() is eng._graphs[True]
+    assert seen == [17, 384] and eng._host_pos == [17] and set(eng._graphs) == {True, False}
+
+
 def test_bench_traffic_is_reported_only_for_the_profiled_source(tmp_path, monkeypatch):
     """A committed PMC traffic figure is used only while the kernel's source file (and
     common.h) hash to the sha recorded when it was measured; otherwise traffic is null and
