@@ -126,6 +126,16 @@ class PrefillPlan:
         self.kexp, self.vexp = kexp, vexp
 
 
+def _row_bounds(lens: list[int], bases: list[int], caps: list[int]) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Position, cache base and capacity of every row of prompts of the given lengths laid one after
+    the other.  Like the upload below it keeps to operations that torch runs on the calling thread up
+    to 32,768 rows: repeat_interleave and indexing start the thread pool for few rows, which kept the
+    host for 5 to 14 ms in 3 of 100 calls (16 threads; a 1,149-token prefill of 2.4 ms)."""
+    return (torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]),
+            torch.cat([torch.full((n,), b, dtype=torch.int64) for n, b in zip(lens, bases)]),
+            torch.cat([torch.full((n,), c, dtype=torch.int32) for n, c in zip(lens, caps)]))
+
+
 def _chunk_segments(lens: list[int], s: int, e: int) -> list[tuple[int, int, int, int]]:
     """(first chunk row, rows, sequence, first position) of each sequence's rows in the chunk of rows
     [s, e) of prompts of the given lengths laid one after the other."""
@@ -194,15 +204,20 @@ class _Upload:
         self.size += -(-t.numel() * t.element_size() // 16) * 16
         return len(self.parts) - 1
 
-    def send(self, device) -> list[torch.Tensor]:
-        """The parts on `device`, in the order they were added."""
-        host = torch.empty(max(self.size, 16), dtype=torch.uint8, pin_memory=True)
+    def fill(self, host: torch.Tensor) -> list[tuple[int, int]]:
+        """The parts one after the other in `host`; the (offset, bytes) of each."""
         at, offs = 0, []
         for t in self.parts:
             n = t.numel() * t.element_size()
-            host[at:at + n].copy_(t.reshape(-1).view(torch.uint8))
+            host[at:at + n].view(t.dtype).copy_(t.reshape(-1))
             offs.append((at, n))
             at += -(-n // 16) * 16
+        return offs
+
+    def send(self, device) -> list[torch.Tensor]:
+        """The parts on `device`, in the order they were added."""
+        host = torch.empty(max(self.size, 16), dtype=torch.uint8, pin_memory=True)
+        offs = self.fill(host)
         dev = host.to(device, non_blocking=True)
         return [dev[o:o + n].view(t.dtype).reshape(t.shape) for (o, n), t in zip(offs, self.parts)]
 
@@ -680,13 +695,9 @@ class DecodeEngine:
         on_host = all(p.device.type == "cpu" for p in prompts)
         if on_host:
             i_ids = up.add(torch.cat([p.reshape(-1).to(torch.int64) for p in prompts]))
-        counts = torch.tensor(lens)
-        i_pos = up.add(torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]))
-        i_base = up.add(torch.repeat_interleave(torch.tensor(bases, dtype=torch.int64), counts))
-        i_cap = up.add(torch.repeat_interleave(
-            torch.tensor([self.cache.capacities[b] for b in slots], dtype=torch.int32), counts))
+        i_pos, i_base, i_cap = (up.add(t) for t in _row_bounds(lens, bases, [self.cache.capacities[b] for b in slots]))
         i_slot = up.add(torch.tensor(slots, dtype=torch.int64))
-        i_lens = up.add(counts.to(torch.int32))
+        i_lens = up.add(torch.tensor(lens, dtype=torch.int32))
         chunks = []
         for s in range(0, total, max_rows):
             e = min(total, s + max_rows)

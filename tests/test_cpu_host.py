@@ -441,6 +441,39 @@ def test_prefill_groups_bound_the_expansion_by_the_rows_attended():
     assert groups == [_group_tiles(_chunk_segments([2048] * 4, 0, 4 * 2048), bases)]
 
 
+def test_prefill_planning_stays_on_the_calling_thread():
+    """The host work of a prefill's row bounds and upload starts no thread pool (whose first use and
+    wake-ups cost milliseconds where CPUs are shared), and gives each row its prompt's values."""
+    import subprocess
+    import sys
+
+    code = """
+import os, sys
+sys.path.insert(0, sys.argv[1])
+import torch
+from dsv2lite.engine import _Upload, _row_bounds
+lens, bases, caps = [4000, 1, 2340, 3000], [64, 5000, 7, 9000], [4100, 9, 2400, 3100]
+threads = lambda: len(os.listdir("/proc/self/task"))
+host = torch.empty(400000, dtype=torch.uint8)
+torch.set_num_threads(4)
+before = threads()
+rows = _row_bounds(lens, bases, caps)
+up = _Upload()
+for t in (*rows, torch.arange(9341), torch.tensor(lens, dtype=torch.int32)):
+    up.add(t)
+offs = up.fill(host)
+assert threads() == before, (before, threads())
+want = [(p, b, c) for n, b, c in zip(lens, bases, caps) for p in range(n)]
+assert [tuple(int(x) for x in r) for r in zip(*rows)] == want
+for t, (at, n) in zip(up.parts, offs):
+    assert at % 16 == 0 and torch.equal(host[at:at + n].view(t.dtype), t)
+"""
+    pkg = os.path.join(ROOT, "flash-deepseek-v2-lite_amd")
+    r = subprocess.run([sys.executable, "-c", code, pkg], capture_output=True, text=True, timeout=300,
+                       env={**os.environ, "OMP_NUM_THREADS": "4"})
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_chunk_segments_equal_the_rows_own_runs():
     """The chunk plan from prompt lengths alone equals the one read off the chunk's per-row
     sequence and position tensors, for every cut of ragged prompts."""
